@@ -882,8 +882,9 @@ def traffic_from_profile(logn, npoly, tile_bits):
 
 
 def modulus_class(q):
-    """The kernels' modulus class: 2 below 2^55, 1 below 2^60, else 0."""
-    return 2 if q < (1 << 55) else 1 if q < (1 << 60) else 0
+    """The kernels' modulus class: 3 below 2^50, 2 below 2^55, 1 below 2^60,
+    else 0."""
+    return 3 if q < (1 << 50) else 2 if q < (1 << 55) else 1 if q < (1 << 60) else 0
 
 
 def _ntt_k1(logn, tb):

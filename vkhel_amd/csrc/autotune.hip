@@ -63,17 +63,21 @@ struct Tuning {
 		hipStream_t s = ctx->stream;
 		state_bytes = handoff_state_bytes(polys);
 		if (!hip_ok(hipMalloc(&data, polys * n * 8), "autotune alloc") ||
-				!hip_ok(hipMalloc(&tw, n * sizeof(ulonglong2)), "autotune alloc") ||
+				!hip_ok(hipMalloc(&tw, 2 * n * (sizeof(ulonglong2) + sizeof(double))),
+					"autotune alloc") ||
 				!hip_ok(hipMalloc(&tasks, polys * sizeof(NttTask)), "autotune alloc") ||
 				!hip_ok(hipMalloc(&state, state_bytes), "autotune alloc") ||
 				!hip_ok(hipEventCreate(&e0), "event") ||
 				!hip_ok(hipEventCreate(&e1), "event"))
 			return release(), vkhel_ext_last_error();
 		k_fill_residues<<<1024, 256, 0, s>>>(data, polys * n, q, logn);
-		std::vector<ulonglong2> htw(n);
-		for (uint64_t i = 0; i < n; i++) {
+		// pairs of both directions, then their doubles (DevTables)
+		std::vector<ulonglong2> htw(3 * n);
+		double *fp = (double *) (htw.data() + 2 * n);
+		for (uint64_t i = 0; i < 2 * n; i++) {
 			const uint64_t w = (0x9e3779b97f4a7c15ull * (i + 1)) % q;
 			htw[i] = make_ulonglong2(w, shoup63_factor(w, q));
+			fp[i] = fp_center(w, q);
 		}
 		NttConsts c{};
 		c.q = q;
@@ -87,16 +91,20 @@ struct Tuning {
 		c.w1n = c.ninv;
 		c.w1n_p = c.ninv_p;
 		small_reduce_consts(q, c.red_shift, c.red_m);
+		c.fq = (double) q;
+		c.fqinv = 1.0 / (double) q;
+		c.fninv = fp_center(c.ninv, q);
+		c.fw1n = fp_center(c.w1n, q);
 		mc = modulus_class(q);
 		DevTables t;
 		t.n = n;
 		t.fwd = tw;
-		t.inv = tw;
+		t.inv = tw + n;
 		t.c = c;
 		std::vector<NttTask> h(polys);
 		for (uint32_t i = 0; i < polys; i++)
 			h[i] = make_task(t, data + i * n, data + i * n, false);
-		if (!hip_ok(hipMemcpyAsync(tw, htw.data(), n * sizeof(ulonglong2),
+		if (!hip_ok(hipMemcpyAsync(tw, htw.data(), htw.size() * sizeof(ulonglong2),
 						hipMemcpyHostToDevice, s), "autotune upload") ||
 				!hip_ok(hipMemcpyAsync(tasks, h.data(), polys * sizeof(NttTask),
 						hipMemcpyHostToDevice, s), "autotune upload") ||

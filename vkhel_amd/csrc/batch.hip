@@ -287,7 +287,7 @@ constexpr uint32_t kGroupByTableLogn = 17;
 static std::vector<Segment> segment(std::vector<NttTask> &tasks,
 		bool by_table) {
 	const auto key = [](const NttTask &k) {
-		return 3 * k.c.logn + (uint32_t) modulus_class(k.c.q);
+		return kClassCount * k.c.logn + (uint32_t) modulus_class(k.c.q);
 	};
 	std::stable_sort(tasks.begin(), tasks.end(),
 			[&](const NttTask &a, const NttTask &b) {

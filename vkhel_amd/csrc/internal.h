@@ -51,12 +51,19 @@ struct NttConsts {
 	// word i becomes (in2[i] - y) * scale_w mod q, scale_wp the packed
 	// Shoup companion of scale_w
 	uint64_t scale_w, scale_wp;
+	// the double-precision class (q < kFpQ): q, 1/q rounded, and ninv and w1n
+	// as centered residues (fp_center)
+	double fq, fqinv, fninv, fw1n;
 	uint32_t bshift;  // bits - 2
 	uint32_t logn;
 };
 
 // Device copy of one vkhel_ntt_tables: twiddles stored as {w, w'} pairs in
 // the reference's bit-reversed index order (roots[m + i] of stage m).
+// Moduli of the double-precision class also have each twiddle as a double,
+// its centered residue, at the same positions: n doubles per direction,
+// forward then inverse, after the 2n pairs (tw_fp finds them from the
+// pairs a task names).
 struct DevTables {
 	uint64_t n = 0;
 	const ulonglong2 *fwd = nullptr;
@@ -149,8 +156,9 @@ struct TableGenArgs {
 void table_gen_args(uint64_t n, uint64_t q, uint64_t w, TableGenArgs &g);
 // Writes both interleaved {w, Shoup companion} tables of n = 2^g.logn
 // entries (the layout tw_pos describes) on stream `st`.
+// and, unless `fp` is null, the 2n doubles of the double-precision class.
 hipError_t launch_gen_tables(const TableGenArgs &g, ulonglong2 *fwd,
-		ulonglong2 *inv, hipStream_t st);
+		ulonglong2 *inv, double *fp, hipStream_t st);
 uint64_t inv_mod_2_64(uint64_t q);
 
 // One polynomial transform for the fused kernel: which words, which
@@ -179,9 +187,26 @@ constexpr uint64_t kNoReduceQ = 1ull << 55;
 // kept below 8q with one reduction per butterfly, inverse below 4q, both
 // with products below 4q (8q < 2^63).
 constexpr uint64_t kMidQ = 1ull << 60;
-enum { kClassGeneral = 0, kClassMid = 1, kClassSmall = 2 };
+// Below this bound the double-precision class: residues are integers held in
+// doubles, products formed exactly by fused multiply-adds (ntt_fp.h), 8
+// full-rate instructions per butterfly against about 16.  8q < 2^53 keeps
+// every sum exact.
+constexpr uint64_t kFpQ = 1ull << 50;
+enum { kClassGeneral = 0, kClassMid = 1, kClassSmall = 2, kClassFp = 3,
+	kClassCount = 4 };
 inline int modulus_class(uint64_t q) {
-	return q < kNoReduceQ ? kClassSmall : q < kMidQ ? kClassMid : kClassGeneral;
+	return q < kFpQ ? kClassFp : q < kNoReduceQ ? kClassSmall
+		: q < kMidQ ? kClassMid : kClassGeneral;
+}
+// The residue of v < q (q odd) in [-(q - 1)/2, (q - 1)/2], exact in a double
+// for q < kFpQ.
+__host__ __device__ inline double fp_center(uint64_t v, uint64_t q) {
+	return v > q / 2 ? -(double) (q - v) : (double) v;
+}
+// The doubles of a direction's twiddles, from its pairs (DevTables).
+__host__ __device__ inline const double *tw_fp(const ulonglong2 *tw,
+		uint64_t n, bool inverse) {
+	return (const double *) (tw + (inverse ? n : 2 * n)) + (inverse ? n : 0);
 }
 
 struct NttTask {

@@ -145,12 +145,29 @@ static bool fused_supported(uint32_t logn) {
 	return logn >= (uint32_t) kMinFusedLogn && logn <= (uint32_t) kMaxFusedLogn;
 }
 
+// Shapes and kernels of tile size TB, entry i serving log2 n = i + 3.
+template <int TB>
+static const std::array<FusedEntry, kFusedEntries> &fused_table() {
+	static const std::array<FusedEntry, kFusedEntries> table = [] {
+		auto t = make_fused_shapes<TB>(
+				std::make_integer_sequence<int, kFusedEntries>());
+		for (int i = 0; i < kFusedEntries; i++) {
+			t[i].k[kClassGeneral] = fused_class_table<TB, kClassGeneral>()[i];
+			t[i].k[kClassMid] = fused_class_table<TB, kClassMid>()[i];
+			t[i].k[kClassSmall] = fused_class_table<TB, kClassSmall>()[i];
+			t[i].k[kClassFp] = fused_class_table<TB, kClassFp>()[i];
+		}
+		return t;
+	}();
+	return table;
+}
+
 // Tile sizes (log2 words) the fused kernels are compiled for.
 static const FusedEntry &fused_entry(uint32_t logn, int tile_bits) {
-	const FusedEntry *t = tile_bits == 11 ? fused_table_kt11()
-		: tile_bits == 12 ? fused_table_kt12() : tile_bits == 13 ? fused_table_kt13()
-		: fused_table_kt14();
-	return t[logn - kMinFusedLogn];
+	const uint32_t i = logn - kMinFusedLogn;
+	return tile_bits == 11 ? fused_table<11>()[i]
+		: tile_bits == 12 ? fused_table<12>()[i]
+		: tile_bits == 13 ? fused_table<13>()[i] : fused_table<14>()[i];
 }
 
 NttTask make_task(const DevTables &t, const uint64_t *in, uint64_t *out,
@@ -251,19 +268,19 @@ static int launch_fused_impl(const vkhel_ctx *ctx, const NttTask &uniform,
 			}
 			// forward: columns, then rows; inverse: rows, then columns
 			if (!inverse) {
-				hipLaunchKernelGGL(e1.fwd_a[s][mc], dim3(e1.tiles, count),
+				hipLaunchKernelGGL(e1.k[mc].fwd_a[s], dim3(e1.tiles, count),
 						dim3(e1.threads), 0, st, u, d, 0u);
-				hipLaunchKernelGGL(e2.fwd_b[s][mc], dim3(e2.tiles, count),
+				hipLaunchKernelGGL(e2.k[mc].fwd_b[s], dim3(e2.tiles, count),
 						dim3(e2.threads), 0, st, u, d, kSecondPass | kReversed);
 			} else {
-				hipLaunchKernelGGL(e2.inv_b[s][mc], dim3(e2.tiles, count),
+				hipLaunchKernelGGL(e2.k[mc].inv_b[s], dim3(e2.tiles, count),
 						dim3(e2.threads), 0, st, u, d, 0u);
-				hipLaunchKernelGGL(e1.inv_a[s][mc], dim3(e1.tiles, count),
+				hipLaunchKernelGGL(e1.k[mc].inv_a[s], dim3(e1.tiles, count),
 						dim3(e1.threads), 0, st, u, d, kSecondPass | kReversed);
 			}
 		}
 	} else {
-		hipLaunchKernelGGL(inverse ? e.inv[mc] : e.fwd[mc],
+		hipLaunchKernelGGL(inverse ? e.k[mc].inv : e.k[mc].fwd,
 				dim3(ntasks), dim3(e.threads), 0, st, uniform, dev_tasks);
 	}
 	return hip_ok(hipGetLastError(), "ntt fused launch") ? VKHEL_OK
@@ -337,7 +354,7 @@ static int launch_handoff(const vkhel_ctx *ctx, const FusedEntry &e,
 	const uint32_t words = handoff_state_words(ntasks);
 	hipLaunchKernelGGL(k_handoff_reset, dim3(std::min<uint32_t>((words + 255) / 256,
 					1024)), dim3(256), 0, st, state, words);
-	const HandoffKernel k = inverse ? e.inv_h[mc] : e.fwd_h[mc];
+	const HandoffKernel k = inverse ? e.k[mc].inv_h : e.k[mc].fwd_h;
 	// one workgroup per ticket: placed round-robin over the XCDs, this grid
 	// gives every XCD as many workgroups as the longest queue (XCD 0's) has
 	// tickets
@@ -411,7 +428,7 @@ static int polymul_impl(const NttTask &ucol_a, const NttTask &ucol_b,
 				"fused polymul: unsupported log2 n = %u on 2^%d tiles", logn,
 				tile_bits);
 	if (e.tiles == 1) {
-		hipLaunchKernelGGL(e.pm[mc], dim3(ntasks), dim3(e.threads), 0, st, upm,
+		hipLaunchKernelGGL(e.k[mc].pm, dim3(ntasks), dim3(e.threads), 0, st, upm,
 				pm_tasks, 0u);
 	} else {
 		// Chunks of 2^24 words per operand, so that the row kernel reads
@@ -427,16 +444,16 @@ static int polymul_impl(const NttTask &ucol_a, const NttTask &ucol_b,
 			const NttTask *pt = pm_tasks ? pm_tasks + first : nullptr;
 			// the forward column passes of a and b
 			if (col_tasks) {
-				hipLaunchKernelGGL(e.fwd_a[0][mc], dim3(e.tiles, 2 * count),
+				hipLaunchKernelGGL(e.k[mc].fwd_a[0], dim3(e.tiles, 2 * count),
 						dim3(e.threads), 0, st, ucol_a, col_tasks + 2 * first, 0u);
 			} else {
-				hipLaunchKernelGGL(e.fwd_a[0][mc], grid, dim3(e.threads), 0, st, ucol_a,
+				hipLaunchKernelGGL(e.k[mc].fwd_a[0], grid, dim3(e.threads), 0, st, ucol_a,
 						(const NttTask *) nullptr, 0u);
-				hipLaunchKernelGGL(e.fwd_a[0][mc], grid, dim3(e.threads), 0, st, ucol_b,
+				hipLaunchKernelGGL(e.k[mc].fwd_a[0], grid, dim3(e.threads), 0, st, ucol_b,
 						(const NttTask *) nullptr, 0u);
 			}
-			hipLaunchKernelGGL(e.pm[mc], grid, dim3(e.threads), 0, st, upm, pt, 0u);
-			hipLaunchKernelGGL(e.inv_a[0][mc], grid, dim3(e.threads), 0, st, upm, pt,
+			hipLaunchKernelGGL(e.k[mc].pm, grid, dim3(e.threads), 0, st, upm, pt, 0u);
+			hipLaunchKernelGGL(e.k[mc].inv_a[0], grid, dim3(e.threads), 0, st, upm, pt,
 					kSecondPass);
 		}
 	}

@@ -8,6 +8,7 @@
 #include "handoff.h"
 #include "internal.h"
 #include "modarith.h"
+#include "ntt_fp.h"
 
 namespace vk {
 
@@ -26,25 +27,28 @@ constexpr uint32_t kSecondPass = 1, kReversed = 2;
 typedef void (*HandoffKernel)(NttTask, const NttTask *, uint32_t, uint32_t *,
 		uint32_t, uint32_t);
 
-// One compiled (log2 n, tile size) variant, per modulus class (index
-// kClassGeneral / kClassMid / kClassSmall, modulus_class()): whole-transform
-// kernels for both directions (one workgroup per polynomial), the two
-// passes as separate kernels (one workgroup per tile: the default for
-// two-pass sizes), and launch shape.
-struct FusedEntry {
-	FusedKernel fwd[3], inv[3];
-	// [split][class]: split 0 takes the top ntt_k1 stages in pass 1, split 1
-	// the top alt_k1 (the same kernels as split 0 where there is none)
-	PassKernel fwd_a[2][3], fwd_b[2][3], inv_b[2][3], inv_a[2][3];
-	// the middle of a polynomial product (k_ntt_pm; pm_ok: this size and
-	// tile allow it)
-	PassKernel pm[3];
-	bool pm_ok;
+// The kernels of one (log2 n, tile size) variant for one modulus class
+// (modulus_class()): whole-transform kernels for both directions (one
+// workgroup per polynomial), the two passes as separate kernels (one
+// workgroup per tile: the default for two-pass sizes).
+struct ClassKernels {
+	FusedKernel fwd, inv;
+	// [split]: split 0 takes the top ntt_k1 stages in pass 1, split 1 the top
+	// alt_k1 (the same kernels as split 0 where there is none)
+	PassKernel fwd_a[2], fwd_b[2], inv_b[2], inv_a[2];
+	// the middle of a polynomial product (k_ntt_pm)
+	PassKernel pm;
 	// one-launch two-pass transforms (two-pass sizes only)
-	HandoffKernel fwd_h[3], inv_h[3];
+	HandoffKernel fwd_h, inv_h;
+};
+
+// One (log2 n, tile size) variant: launch shape and each class's kernels.
+struct FusedEntry {
+	bool pm_ok;  // this size and tile allow the fused product kernel
 	int threads;
 	int tiles;  // tiles per pass (1: one-tile size, passes unused)
 	int k1[2];  // stages of pass 1 per split choice (0 for one-tile sizes)
+	ClassKernels k[kClassCount];
 };
 
 constexpr int kMaxFusedLogn = 20;
@@ -378,6 +382,7 @@ typedef __attribute__((address_space(1))) uint64_t gu64;
 typedef __attribute__((address_space(1))) const uint64_t gcu64;
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(1))) const u64x2 gcu128;
+typedef __attribute__((address_space(1))) const double gcdouble;
 
 // Word indices within one polynomial stay below 2^28, so the byte offset
 // is formed in 32 bits: the compiler then addresses with the wave-uniform
@@ -413,6 +418,10 @@ __device__ __forceinline__ ulonglong2 gload_tw(const ulonglong2 *p,
 		uint32_t i) {
 	const u64x2 v = *(gcu128 *) ((gcchar *) p + (i << 4));
 	return make_ulonglong2(v.x, v.y);
+}
+
+__device__ __forceinline__ double gload_tw(const double *p, uint32_t i) {
+	return *(gcdouble *) ((gcchar *) p + (i << 3));
 }
 
 // One padding word per 8 keeps the radix-8 access patterns conflict free.
@@ -455,10 +464,31 @@ __host__ __device__ constexpr int tw_slot(int d, int gi) {
 	return (d == 2 ? 0 : d == 1 ? 1 : 3) + gi;
 }
 
-// Loads every twiddle pair round R uses into w (slots as tw_slot).
-template <class G, bool INV, int R, int LOGN>
-__device__ __forceinline__ void load_round_tw(ulonglong2 w[7], uint32_t t,
-		uint32_t gbase, const ulonglong2 *tw) {
+// A class's twiddle: a {w, Shoup companion} pair, or a double.
+template <int MC>
+using Twiddle = std::conditional_t<MC == kClassFp, double, ulonglong2>;
+
+// A direction's twiddles of an n-word transform for a class, with the pairs
+// they come from.
+template <int MC>
+struct Twiddles {
+	const Twiddle<MC> *p;
+	const ulonglong2 *pairs;
+};
+
+template <int MC, bool INV>
+__device__ __forceinline__ Twiddles<MC> twiddles(const ulonglong2 *tw,
+		uint32_t n) {
+	if constexpr (MC == kClassFp)
+		return Twiddles<MC>{tw_fp(tw, n, INV), tw};
+	else
+		return Twiddles<MC>{tw, tw};
+}
+
+// Loads every twiddle round R uses into w (slots as tw_slot).
+template <class G, bool INV, int R, int LOGN, class T>
+__device__ __forceinline__ void load_round_tw(T w[7], uint32_t t,
+		uint32_t gbase, const T *tw) {
 	using RD = Round<G, INV, R>;
 	constexpr int F = RD::F;
 	const uint32_t l0 = round_base<F>(t);
@@ -573,6 +603,195 @@ constexpr bool round_wave_local() {
 // whatever the pass.
 enum { kIoPreloaded = 1, kIoKeep = 2, kIoStreamIn = 4 };
 
+// True for the pass of a transform that reads its input / writes its result.
+template <class G, bool INV>
+constexpr bool reads_input() {
+	return G::P == 0 || G::P == (INV ? 2 : 1);
+}
+template <class G, bool INV>
+constexpr bool writes_result() {
+	return G::P == 0 || G::P == (INV ? 1 : 2);
+}
+
+template <class G, bool INV, int R>
+constexpr int round_stages() {
+	return Round<G, INV, R>::BHI - Round<G, INV, R>::BLO;
+}
+
+// The double-precision class's forward values before round R, in units of
+// q/1024: canonical input below q, and a round whose growth would pass 8q
+// starts by reducing every value (fp_forward_reduces).
+template <class G, int R>
+constexpr int fp_forward_bound();
+template <class G, int R>
+constexpr bool fp_forward_reduces() {
+	return fp_grow(fp_forward_bound<G, R>(), round_stages<G, false, R>()) >
+		kFpLimit;
+}
+template <class G, int R>
+constexpr int fp_forward_bound() {
+	if constexpr (R == 0)
+		return reads_input<G, false>() ? 1024 : kFpForwardPass;
+	else
+		return fp_grow(fp_forward_reduces<G, R - 1>() ? kFpReduced
+				: fp_forward_bound<G, R - 1>(), round_stages<G, false, R - 1>());
+}
+
+// The butterflies of round R for the double-precision class on v's eight
+// words, which hold input words (a pass that reads the input; PRE: already
+// doubles) or doubles of any sign, and leave result words or doubles (KEEP:
+// doubles).  At most 8 instructions per butterfly and three per value where
+// a bound calls for a reduction (about one reduction per two rounds forward,
+// four of eight values per round inverse).
+template <class G, bool INV, int R, int LOGN, bool PRE, bool KEEP>
+__device__ __forceinline__ void fp_round(uint64_t v[8], const double w[7],
+		const ulonglong2 *tw, const NttConsts &c) {
+#pragma clang fp contract(off)
+	using RD = Round<G, INV, R>;
+	constexpr int F = RD::F;
+	constexpr int ACTIVE = (F >= RD::BLO && F < RD::BHI ? 1 : 0) |
+		(F + 1 >= RD::BLO && F + 1 < RD::BHI ? 2 : 0) |
+		(F + 2 >= RD::BLO && F + 2 < RD::BHI ? 4 : 0);
+	constexpr bool LAST_ROUND = R == G::ROUNDS - 1;
+	constexpr bool FIRST = R == 0 && reads_input<G, INV>() && !PRE;
+	constexpr bool RESULT = LAST_ROUND && writes_result<G, INV>() && !KEEP;
+	const FpK k{c.fq, c.fqinv};
+	double x[8];
+	if constexpr (FIRST && !INV) {
+		// Words below q convert as they are.  A wave holding a larger one
+		// reduces them all, exactly while they are below 2^52 (where the
+		// reference's 64-bit sum X + WY cannot wrap), and otherwise takes the
+		// reference's first stage in integers (bf_fwd_first) up to the
+		// stage's outputs.
+		bool canon = true;
+		uint32_t top = 0;
+#pragma unroll
+		for (int e = 0; e < 8; e++) {
+			canon &= v[e] < c.q;
+			top |= (uint32_t) (v[e] >> 32);
+		}
+		bool staged = false;
+		if (__all(canon)) {
+#pragma unroll
+			for (int e = 0; e < 8; e++)
+				x[e] = fp_from_word(v[e]);
+		} else if (__all(top < (1u << 20))) {
+#pragma unroll
+			for (int e = 0; e < 8; e++)
+				x[e] = fp_reduce(fp_from_word(v[e]), k);
+		} else {
+			const ulonglong2 w1 = gload_tw(tw, 1);
+#pragma unroll
+			for (int e = 0; e < 4; e++)
+				bf_fwd_first(v[e], v[e + 4], w1, c);
+#pragma unroll
+			for (int e = 0; e < 8; e++)
+				x[e] = fp_from_word(v[e]);
+			staged = true;
+		}
+		if (!staged) {
+#pragma unroll
+			for (int e = 0; e < 4; e++) {
+				const double t = fp_mulmod(x[e + 4], w[0], k);
+				x[e + 4] = x[e] - t;
+				x[e] = x[e] + t;
+			}
+		}
+	} else if constexpr (FIRST) {
+#pragma unroll
+		for (int e = 0; e < 8; e++)
+			x[e] = fp_from_word(v[e]);
+	} else {
+#pragma unroll
+		for (int e = 0; e < 8; e++)
+			x[e] = __builtin_bit_cast(double, v[e]);
+	}
+
+	if constexpr (!INV) {
+		if constexpr (fp_forward_reduces<G, R>()) {
+#pragma unroll
+			for (int e = 0; e < 8; e++)
+				x[e] = fp_reduce(x[e], k);
+		}
+#pragma unroll
+		for (int d = 2; d >= 0; d--) {
+			if (!((ACTIVE >> d) & 1) || (FIRST && F + d + G::SHIFT == LOGN - 1))
+				continue;
+#pragma unroll
+			for (int gi = 0; gi < (4 >> d); gi++) {
+#pragma unroll
+				for (int li = 0; li < (1 << d); li++) {
+					const int e = (gi << (d + 1)) | li, f = e | (1 << d);
+					const double t = fp_mulmod(x[f], w[tw_slot(d, gi)], k);
+					x[f] = x[e] - t;
+					x[e] = x[e] + t;
+				}
+			}
+		}
+		constexpr int BOUND = fp_grow(fp_forward_reduces<G, R>() ? kFpReduced
+				: fp_forward_bound<G, R>(), round_stages<G, INV, R>());
+		static_assert(BOUND <= kFpLimit, "forward values past 8q");
+		if constexpr (LAST_ROUND && !writes_result<G, INV>() &&
+				BOUND > kFpForwardPass) {
+#pragma unroll
+			for (int e = 0; e < 8; e++)
+				x[e] = fp_reduce(x[e], k);
+		}
+	} else {
+		constexpr int TOP = LOGN - 1 - G::SHIFT - F;  // register bit of the last stage
+		constexpr bool HAS_LAST = TOP >= 0 && TOP <= 2 && ((ACTIVE >> TOP) & 1);
+		constexpr FpInvPlan plan = fp_inv_plan(FIRST ? 1024 : kFpInverseRound,
+				ACTIVE, RESULT);
+#pragma unroll
+		for (int d = 0; d < 3; d++) {
+			if (!((ACTIVE >> d) & 1))
+				continue;
+#pragma unroll
+			for (int e = 0; e < 8; e++) {
+				if ((plan.before[d] >> e) & 1)
+					x[e] = fp_reduce(x[e], k);
+			}
+#pragma unroll
+			for (int e = 0; e < 8; e++) {
+				if ((e >> d) & 1)
+					continue;
+				const int f = e | (1 << d);
+				const double s = x[e] + x[f], t = x[e] - x[f];
+				if (HAS_LAST && d == TOP) {
+					// n^-1 folded into the last stage (src/vector.c:633-638)
+					x[e] = fp_mulmod(s, c.fninv, k);
+					x[f] = fp_mulmod(t, c.fw1n, k);
+				} else {
+					x[e] = s;
+					x[f] = fp_mulmod(t, w[tw_slot(d, e >> (d + 1))], k);
+				}
+			}
+		}
+#pragma unroll
+		for (int e = 0; e < 8; e++) {
+			if ((plan.after >> e) & 1)
+				x[e] = fp_reduce(x[e], k);
+		}
+	}
+
+	if constexpr (RESULT) {
+#pragma unroll
+		for (int e = 0; e < 8; e++)
+			v[e] = fp_canonical(x[e], k);
+		if constexpr (INV) {
+			if (c.post_p) {
+#pragma unroll
+				for (int e = 0; e < 8; e++)
+					v[e] = post_center(v[e], c);
+			}
+		}
+	} else {
+#pragma unroll
+		for (int e = 0; e < 8; e++)
+			v[e] = __builtin_bit_cast(uint64_t, x[e]);
+	}
+}
+
 // Tiles of 2^14 words have 2048 threads' worth of work (8 words each) but
 // a workgroup holds at most 1024: physical thread tp then runs the round's
 // work of virtual threads tp and tp + 1024 one after the other (G::VT).
@@ -581,9 +800,9 @@ enum { kIoPreloaded = 1, kIoKeep = 2, kIoStreamIn = 4 };
 // exchange rules above hold unchanged; the synchronisations of a round
 // come after all its virtual threads.
 template <class G, bool INV, int R, int LOGN, bool TRAIL, int MC, int IO = 0>
-__device__ __forceinline__ void run_round(uint64_t v[8], ulonglong2 w[7],
+__device__ __forceinline__ void run_round(uint64_t v[8], Twiddle<MC> w[7],
 		uint32_t tp, const uint64_t *src, const uint64_t *src2, uint64_t *dst,
-		uint64_t *lds, uint32_t jbase, uint32_t gbase, const ulonglong2 *tw,
+		uint64_t *lds, uint32_t jbase, uint32_t gbase, const Twiddles<MC> &tw,
 		const NttConsts &c, bool final) {
 	using RD = Round<G, INV, R>;
 	constexpr int F = RD::F;
@@ -672,11 +891,14 @@ __device__ __forceinline__ void run_round(uint64_t v[8], ulonglong2 w[7],
 			// every twiddle of the round, issued before any arithmetic
 			// (loading the next round's before the barrier instead costs
 			// registers beyond eight waves per SIMD and measured no faster)
-			load_round_tw<G, INV, R, LOGN>(w, t, gbase, tw);
+			load_round_tw<G, INV, R, LOGN>(w, t, gbase, tw.p);
 		}
 
 		// ---- butterflies ----
-		if (active) {
+		if constexpr (MC == kClassFp) {
+			if (active)
+				fp_round<G, INV, R, LOGN, PRE, KEEP>(v, w, tw.pairs, c);
+		} else if (active) {
 			const LazyK lk = lazy_consts(c);
 			// inverse with deferred sum reductions (q < kNoReduceQ): stages
 			// present in this round, and the bound its inputs enter with
@@ -871,8 +1093,8 @@ template <class G, bool INV, int LOGN, bool TRAIL, int MC, int IO, int... R>
 __device__ __forceinline__ void run_rounds_v(std::integer_sequence<int, R...>,
 		uint64_t v[8], uint32_t t, const uint64_t *src, const uint64_t *src2,
 		uint64_t *dst, uint64_t *lds, uint32_t jbase, uint32_t gbase,
-		const ulonglong2 *tw, const NttConsts &c, bool final) {
-	ulonglong2 w[7];
+		const Twiddles<MC> &tw, const NttConsts &c, bool final) {
+	Twiddle<MC> w[7];
 	(run_round<G, INV, R, LOGN, TRAIL, MC, IO>(v, w, t, src, src2, dst, lds,
 			jbase, gbase, tw, c, final), ...);
 }
@@ -880,7 +1102,7 @@ __device__ __forceinline__ void run_rounds_v(std::integer_sequence<int, R...>,
 template <class G, bool INV, int LOGN, bool TRAIL, int MC, int... R>
 __device__ __forceinline__ void run_rounds(std::integer_sequence<int, R...> seq,
 		uint32_t t, const uint64_t *src, const uint64_t *src2, uint64_t *dst,
-		uint64_t *lds, uint32_t jbase, uint32_t gbase, const ulonglong2 *tw,
+		uint64_t *lds, uint32_t jbase, uint32_t gbase, const Twiddles<MC> &tw,
 		const NttConsts &c, bool final) {
 	uint64_t v[8];
 	run_rounds_v<G, INV, LOGN, TRAIL, MC, 0>(seq, v, t, src, src2, dst, lds,
@@ -889,9 +1111,10 @@ __device__ __forceinline__ void run_rounds(std::integer_sequence<int, R...> seq,
 
 template <int LOGN, int PASS, int TB, bool INV, int MC>
 __device__ __forceinline__ void run_pass(const uint64_t *src,
-		const uint64_t *src2, uint64_t *dst, uint64_t *lds, const ulonglong2 *tw,
-		const NttConsts &c, bool final) {
+		const uint64_t *src2, uint64_t *dst, uint64_t *lds,
+		const ulonglong2 *pairs, const NttConsts &c, bool final) {
 	using G = Geo<LOGN, PASS, TB>;
+	const auto tw = twiddles<MC, INV>(pairs, 1u << LOGN);
 	const uint32_t t = threadIdx.x;
 	for (uint32_t i = 0; i < (uint32_t) G::NTILES; i++) {
 		// pass 1 tiles start at column i * 2^cb; pass 2 tiles at row block
@@ -998,7 +1221,7 @@ __attribute__((amdgpu_waves_per_eu(pass_waves(LOGN, PASS, TB)))) void k_ntt_pass
 		run_rounds<G, INV, LOGN, false, MC>(
 				std::make_integer_sequence<int, G::ROUNDS>(), threadIdx.x,
 				second ? k.out : k.in, with_in2 ? k.in2 : nullptr, k.out, lds, jbase,
-				gbase, k.tw, k.c, second);
+				gbase, twiddles<MC, INV>(k.tw, 1u << LOGN), k.c, second);
 	}
 }
 
@@ -1080,13 +1303,14 @@ __attribute__((amdgpu_waves_per_eu(pass_waves(LOGN, 1, TB)))) void k_ntt_handoff
 			const uint32_t jb = w.tile << TB;
 			run_rounds<G2, INV, LOGN, false, MC>(
 					std::make_integer_sequence<int, G2::ROUNDS>(), t,
-					w.producer ? tk.in : tk.out, tk.in2, tk.out, lds, jb, jb, tk.tw,
-					tk.c, !w.producer);
+					w.producer ? tk.in : tk.out, tk.in2, tk.out, lds, jb, jb,
+					twiddles<MC, INV>(tk.tw, 1u << LOGN), tk.c, !w.producer);
 		} else {
 			run_rounds<G1, INV, LOGN, false, MC>(
 					std::make_integer_sequence<int, G1::ROUNDS>(), t,
 					w.producer ? tk.in : tk.out, nullptr, tk.out, lds,
-					w.tile << G1::CB, 0, tk.tw, tk.c, !w.producer);
+					w.tile << G1::CB, 0, twiddles<MC, INV>(tk.tw, 1u << LOGN), tk.c,
+					!w.producer);
 		}
 		if (w.producer) {
 			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1167,71 +1391,87 @@ __attribute__((amdgpu_waves_per_eu(pm_waves(LOGN, TB)))) void k_ntt_pm(
 		// leave the L2 to the two twiddle tables the kernel rereads (2^15 to
 		// 2^17 measured 1.5-3% faster than with ordinary loads).
 		uint64_t vb[8], v[8];
+		const auto fwd = twiddles<MC, false>(k.tw2, 1u << LOGN);
 		run_rounds_v<G, false, LOGN, false, MC, kIoKeep | kIoStreamIn>(seq, vb, t, k.in2,
-				nullptr, k.out, lds, jbase, jbase, k.tw2, k.c, true);
+				nullptr, k.out, lds, jbase, jbase, fwd, k.c, true);
 		// (a's first round may write LDS words other waves read in b's last)
 		__syncthreads();
 		run_rounds_v<G, false, LOGN, false, MC, kIoKeep | kIoStreamIn>(seq, v, t, k.in,
-				nullptr, k.out, lds, jbase, jbase, k.tw2, k.c, true);
+				nullptr, k.out, lds, jbase, jbase, fwd, k.c, true);
 		if (G::THREADS >= 64 || t < (uint32_t) G::THREADS) {
 #pragma unroll
-			for (int e = 0; e < 8; e++)
-				v[e] = spectra_product(v[e], vb[e], k.c);
+			for (int e = 0; e < 8; e++) {
+				if constexpr (MC == kClassFp) {
+					// both spectra are doubles below 8q here; one operand of a
+					// product has to be below q/2
+					const FpK fk{k.c.fq, k.c.fqinv};
+					v[e] = __builtin_bit_cast(uint64_t, fp_mulmod(
+							__builtin_bit_cast(double, v[e]), fp_reduce(
+								__builtin_bit_cast(double, vb[e]), fk), fk));
+				} else {
+					v[e] = spectra_product(v[e], vb[e], k.c);
+				}
+			}
 		}
 		wave_sync();
 		run_rounds_v<G, true, LOGN, false, MC, kIoPreloaded>(seq, v, t, nullptr,
-				nullptr, k.out, lds, jbase, jbase, k.tw, k.c, PASS == 0);
+				nullptr, k.out, lds, jbase, jbase,
+				twiddles<MC, true>(k.tw, 1u << LOGN), k.c, PASS == 0);
 	}
 }
 
-// The pass kernels of one (size, pass, direction, tile, split) for the
-// three modulus classes; the alternative split is instantiated only where
-// it exists (ALT_SPLIT: 1 there, else 0, naming the default kernels).
-#define PASS_ROW(LG, PS, INV, TB, SP) \
-	{k_ntt_pass<LG, PS, INV, TB, 0, SP>, k_ntt_pass<LG, PS, INV, TB, 1, SP>, \
-		k_ntt_pass<LG, PS, INV, TB, 2, SP>}
-#define ALT_SPLIT(LG, TB) (alt_k1(LG, TB) > 0 ? 1 : 0)
+// The pass kernels of one (size, pass, direction, tile) for both splits;
+// the alternative split is instantiated only where it exists (else it names
+// the default kernel).
+template <int LG, int TB, int MC, int PS, bool INV>
+constexpr void set_passes(PassKernel k[2]) {
+	k[0] = k_ntt_pass<LG, PS, INV, TB, MC, 0>;
+	k[1] = k_ntt_pass<LG, PS, INV, TB, MC, (alt_k1(LG, TB) > 0 ? 1 : 0)>;
+}
 
-// Kernel table for tile size TB, entry i serving log2 n = i + 3.
+// The whole-polynomial two-pass kernels and the one-launch ones are tuning
+// modes that measured slower than the split passes at every size: moduli of
+// the double-precision class run the small class's there.
+template <int LG, int TB, int MC>
+constexpr ClassKernels class_kernels() {
+	constexpr int MC2 = MC == kClassFp ? (int) kClassSmall : MC;
+	constexpr int MC1 = LG <= TB ? MC : MC2;
+	ClassKernels k{};
+	k.fwd = k_ntt_fused<LG, false, TB, MC1>;
+	k.inv = k_ntt_fused<LG, true, TB, MC1>;
+	set_passes<LG, TB, MC, 1, false>(k.fwd_a);
+	set_passes<LG, TB, MC, 2, false>(k.fwd_b);
+	set_passes<LG, TB, MC, 2, true>(k.inv_b);
+	set_passes<LG, TB, MC, 1, true>(k.inv_a);
+	k.pm = k_ntt_pm<LG, TB, MC>;
+	k.fwd_h = k_ntt_handoff<LG, false, TB, MC2>;
+	k.inv_h = k_ntt_handoff<LG, true, TB, MC2>;
+	return k;
+}
+
+// Kernels of tile size TB and class MC, entry i serving log2 n = i + 3.
+template <int TB, int MC, int... L>
+constexpr std::array<ClassKernels, sizeof...(L)> make_class_table(
+		std::integer_sequence<int, L...>) {
+	return {class_kernels<L + kMinFusedLogn, TB, MC>()...};
+}
+
+// One translation unit per tile size and class instantiates these
+// (ntt_fused_inst.hip).  Sizes n <= 2^TB use the one-tile kernel and are
+// identical across tiles.
+template <int TB, int MC>
+const ClassKernels *fused_class_table();
+
+// Launch shapes of tile size TB.
 template <int TB, int... L>
-constexpr std::array<FusedEntry, sizeof...(L)> make_fused_table(
+constexpr std::array<FusedEntry, sizeof...(L)> make_fused_shapes(
 		std::integer_sequence<int, L...>) {
 	return {FusedEntry{
-		{k_ntt_fused<L + kMinFusedLogn, false, TB, 0>,
-			k_ntt_fused<L + kMinFusedLogn, false, TB, 1>,
-			k_ntt_fused<L + kMinFusedLogn, false, TB, 2>},
-		{k_ntt_fused<L + kMinFusedLogn, true, TB, 0>,
-			k_ntt_fused<L + kMinFusedLogn, true, TB, 1>,
-			k_ntt_fused<L + kMinFusedLogn, true, TB, 2>},
-		{PASS_ROW(L + kMinFusedLogn, 1, false, TB, 0),
-			PASS_ROW(L + kMinFusedLogn, 1, false, TB, ALT_SPLIT(L + kMinFusedLogn, TB))},
-		{PASS_ROW(L + kMinFusedLogn, 2, false, TB, 0),
-			PASS_ROW(L + kMinFusedLogn, 2, false, TB, ALT_SPLIT(L + kMinFusedLogn, TB))},
-		{PASS_ROW(L + kMinFusedLogn, 2, true, TB, 0),
-			PASS_ROW(L + kMinFusedLogn, 2, true, TB, ALT_SPLIT(L + kMinFusedLogn, TB))},
-		{PASS_ROW(L + kMinFusedLogn, 1, true, TB, 0),
-			PASS_ROW(L + kMinFusedLogn, 1, true, TB, ALT_SPLIT(L + kMinFusedLogn, TB))},
-		{k_ntt_pm<L + kMinFusedLogn, TB, 0>,
-			k_ntt_pm<L + kMinFusedLogn, TB, 1>,
-			k_ntt_pm<L + kMinFusedLogn, TB, 2>},
 		pm_fusable<L + kMinFusedLogn, TB>(),
-		{k_ntt_handoff<L + kMinFusedLogn, false, TB, 0>,
-			k_ntt_handoff<L + kMinFusedLogn, false, TB, 1>,
-			k_ntt_handoff<L + kMinFusedLogn, false, TB, 2>},
-		{k_ntt_handoff<L + kMinFusedLogn, true, TB, 0>,
-			k_ntt_handoff<L + kMinFusedLogn, true, TB, 1>,
-			k_ntt_handoff<L + kMinFusedLogn, true, TB, 2>},
 		FusedShape<L + kMinFusedLogn, TB>::THREADS,
 		1 << (L + kMinFusedLogn > TB ? L + kMinFusedLogn - TB : 0),
 		{ntt_k1(L + kMinFusedLogn, TB),
-			split_k1(L + kMinFusedLogn, TB, 1)}}...};
+			split_k1(L + kMinFusedLogn, TB, 1)}, {}}...};
 }
-
-// Per-tile-size tables (ntt_fused_kt*.hip).  Sizes n <= 2^TB use the
-// one-tile kernel and are identical across tables.
-const FusedEntry *fused_table_kt11();
-const FusedEntry *fused_table_kt12();
-const FusedEntry *fused_table_kt13();
-const FusedEntry *fused_table_kt14();
 
 }  // namespace vk

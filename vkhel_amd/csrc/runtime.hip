@@ -70,13 +70,15 @@ const DevTables *device_tables(vkhel_ctx *ctx, const vkhel_ntt_tables *t) {
 	table_gen_args(n, q, t->w, ga);
 	DevTables *d = new DevTables;
 	d->n = n;
-	if (!hip_ok(hipMalloc(&d->alloc, 2 * n * sizeof(ulonglong2)),
-				"hipMalloc(tables)")) {
+	const bool fp = q < kFpQ;
+	if (!hip_ok(hipMalloc(&d->alloc, 2 * n * (sizeof(ulonglong2) +
+						(fp ? sizeof(double) : 0))), "hipMalloc(tables)")) {
 		delete d;
 		return nullptr;
 	}
 	ulonglong2 *dev = (ulonglong2 *) d->alloc;
-	if (!hip_ok(launch_gen_tables(ga, dev, dev + n, ctx->table_stream),
+	if (!hip_ok(launch_gen_tables(ga, dev, dev + n,
+					fp ? (double *) (dev + 2 * n) : nullptr, ctx->table_stream),
 				"table generation") ||
 			!hip_ok(hipStreamSynchronize(ctx->table_stream),
 				"table generation sync")) {
@@ -99,6 +101,12 @@ const DevTables *device_tables(vkhel_ctx *ctx, const vkhel_ntt_tables *t) {
 	c.w1n = mulmod_exact(ga.wipow[ga.logn - 1], c.ninv, q);
 	c.w1n_p = shoup63_factor(c.w1n, q);
 	small_reduce_consts(q, c.red_shift, c.red_m);
+	if (fp) {
+		c.fq = (double) q;
+		c.fqinv = 1.0 / (double) q;
+		c.fninv = fp_center(c.ninv, q);
+		c.fw1n = fp_center(c.w1n, q);
+	}
 	ctx->tables.emplace(t->id, d);
 	return d;
 }

@@ -44,9 +44,10 @@ __device__ __forceinline__ uint64_t gen_shoup63(uint64_t r,
 
 // One thread per reference index k in [0, n): writes {w^e, companion} and
 // {w^-e, companion} at the interleaved position of k (tw_pos).  Position 0,
-// which no transform reads, receives w^0.
+// which no transform reads, receives w^0.  The double-precision class's
+// tables (fp, unless null) take the centered residues at the same positions.
 __global__ __launch_bounds__(256) void k_gen_tables(TableGenArgs g,
-		ulonglong2 *fwd, ulonglong2 *inv) {
+		ulonglong2 *fwd, ulonglong2 *inv, double *fp) {
 	const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
 	if (k >= (1u << g.logn))
 		return;
@@ -63,6 +64,10 @@ __global__ __launch_bounds__(256) void k_gen_tables(TableGenArgs g,
 	const uint32_t p = k ? tw_pos(m, k - m) : 0;
 	fwd[p] = make_ulonglong2(r, gen_shoup63(r, g));
 	inv[p] = make_ulonglong2(ri, gen_shoup63(ri, g));
+	if (fp) {
+		fp[p] = fp_center(r, g.q);
+		fp[(1u << g.logn) + p] = fp_center(ri, g.q);
+	}
 }
 
 void table_gen_args(uint64_t n, uint64_t q, uint64_t w, TableGenArgs &g) {
@@ -83,10 +88,10 @@ void table_gen_args(uint64_t n, uint64_t q, uint64_t w, TableGenArgs &g) {
 }
 
 hipError_t launch_gen_tables(const TableGenArgs &g, ulonglong2 *fwd,
-		ulonglong2 *inv, hipStream_t st) {
+		ulonglong2 *inv, double *fp, hipStream_t st) {
 	const uint32_t n = 1u << g.logn;
 	hipLaunchKernelGGL(k_gen_tables, dim3((n + 255) / 256), dim3(256), 0, st,
-			g, fwd, inv);
+			g, fwd, inv, fp);
 	return hipGetLastError();
 }
 
