@@ -197,9 +197,9 @@ static bool check_vectors(const char *fn, bool binary, const vkhel_vector *a,
 	return true;
 }
 
-static void finish(vkhel_ctx *ctx, int rc) {
+static void finish(const vkhel_vector *res, int rc) {
 	if (rc == VKHEL_OK)
-		hip_ok(hipStreamSynchronize(ctx->stream), "sync");
+		(void) wait_call(res->ctx, res->length);
 }
 
 }  // namespace vk
@@ -216,7 +216,7 @@ void vkhel_vector_elemfma(const struct vkhel_vector *a,
 		return;
 	if (mod < 2)
 		return (void) fail(VKHEL_ERR_INVALID, "elemfma: mod must be >= 2");
-	finish(res->ctx, launch_elemfma(a->dev, b->dev, res->dev, res->length,
+	finish(res, launch_elemfma(a->dev, b->dev, res->dev, res->length,
 				multiplier, mod, res->ctx->stream));
 }
 
@@ -236,7 +236,7 @@ void vkhel_vector_elemmod(const struct vkhel_vector *a,
 			(uint32_t) (bitlen(mod) - 2)};
 		rc = launch_unary(a->dev, res->dev, res->length, op, res->ctx->stream);
 	}
-	finish(res->ctx, rc);
+	finish(res, rc);
 }
 
 // src/vector.c:388-427, push constants src/kernels/elemmul.c:159-168.
@@ -246,7 +246,7 @@ void vkhel_vector_elemmul(const struct vkhel_vector *a,
 		return;
 	if (mod < 2)
 		return (void) fail(VKHEL_ERR_INVALID, "elemmul: mod must be >= 2");
-	finish(res->ctx, launch_elemmul(a->dev, b->dev, res->dev, res->length, mod,
+	finish(res, launch_elemmul(a->dev, b->dev, res->dev, res->length, mod,
 				res->ctx->stream));
 }
 
@@ -255,7 +255,7 @@ void vkhel_vector_elemgtadd(const struct vkhel_vector *a,
 		struct vkhel_vector *res, uint64_t bound, uint64_t diff) {
 	if (!check_vectors("elemgtadd", false, a, nullptr, res))
 		return;
-	finish(res->ctx, launch_unary(a->dev, res->dev, res->length,
+	finish(res, launch_unary(a->dev, res->dev, res->length,
 				OpGtAdd{bound, diff}, res->ctx->stream));
 }
 
@@ -268,7 +268,7 @@ void vkhel_vector_elemgtsub(const struct vkhel_vector *a,
 		return (void) fail(VKHEL_ERR_INVALID, "elemgtsub: mod must be >= 2");
 	const OpGtSub op{bound, diff, mod, barrett_mu(mod),
 		(uint32_t) (bitlen(mod) - 2)};
-	finish(res->ctx, launch_unary(a->dev, res->dev, res->length, op,
+	finish(res, launch_unary(a->dev, res->dev, res->length, op,
 				res->ctx->stream));
 }
 

@@ -115,6 +115,12 @@ struct vkhel_ctx {
 	// (handoff.h; 0: from the occupancy).
 	int handoff_ahead = 0;
 
+	// Completion of the synchronous calls (wait_call): a page-locked word that
+	// a kernel enqueued after a call's work sets to the call's number.
+	uint64_t *done = nullptr;
+	std::mutex done_mu;  // orders numbers as the stream sees them
+	uint64_t done_next = 0;
+
 	std::mutex mu;  // guards `tables` (batch and serve threads share it)
 	std::unordered_map<uint64_t, vk::DevTables *> tables;
 	// Page-locked staging buffers of vkhel_vector_map, reused: a map takes
@@ -140,6 +146,11 @@ struct vkhel_vector {
 };
 
 namespace vk {
+
+// Waits for what the calling thread has enqueued on the context's stream, the
+// end of every synchronous call; `words` is how many the call computed.
+// Returns a vkhel_status.
+int wait_call(vkhel_ctx *ctx, uint64_t words);
 
 // Device tables of `t` on `ctx`, generated on the GPU on first use.
 // nullptr on failure (error recorded).

@@ -516,7 +516,7 @@ static void transform(const vkhel_vector *op, vkhel_vector *res,
 		return;
 	if (launch_ntt(ctx, *t, op->dev, res->dev, 1, inverse, ctx->stream) ==
 			VKHEL_OK)
-		hip_ok(hipStreamSynchronize(ctx->stream), "sync");
+		(void) wait_call(ctx, ntt->n);
 }
 
 }  // namespace vk
