@@ -1164,6 +1164,7 @@ __attribute__((amdgpu_waves_per_eu(fused_waves(LOGN, TB)))) void k_ntt_fused(
 		if (k.in2)
 			k.in2 += off;
 	}
+	ieee_mode_off(k.c.q, k.c.two_q);
 	if constexpr (LOGN <= TB) {
 		run_pass<LOGN, 0, TB, INV, MC>(k.in, k.in2, k.out, lds, k.tw, k.c, true);
 	} else if constexpr (!INV) {
@@ -1211,6 +1212,7 @@ __attribute__((amdgpu_waves_per_eu(pass_waves(LOGN, PASS, TB)))) void k_ntt_pass
 			if (k.in2)
 				k.in2 += off;
 		}
+		ieee_mode_off(k.c.q, k.c.two_q);
 		using G = Geo<LOGN, PASS, TB, SPLIT>;
 		const uint32_t i = blockIdx.x;
 		const uint32_t jbase = PASS == 1 ? i << G::CB : i << TB;
@@ -1280,7 +1282,8 @@ __attribute__((amdgpu_waves_per_eu(pass_waves(LOGN, 1, TB)))) void k_ntt_handoff
 		const HandoffWork w = handoff_decode(k, x, npoly, T, ahead);
 		uint32_t *count = state + kHandoffCounts + x * handoff_count_stride(npoly) +
 			w.poly / kXcds;
-		const NttTask tk = tasks[w.poly];
+		NttTask tk = tasks[w.poly];
+		ieee_mode_off(tk.c.q, tk.c.two_q);
 		if (!w.producer) {
 			// (once any wait has given up, none waits again)
 			if (t == 0 && !atomic_peek(state + kHandoffErr)) {
@@ -1382,6 +1385,7 @@ __attribute__((amdgpu_waves_per_eu(pm_waves(LOGN, TB)))) void k_ntt_pm(
 			k.out += off;
 			k.in2 += off;
 		}
+		ieee_mode_off(k.c.q, k.c.two_q);
 		const uint32_t t = threadIdx.x;
 		const uint32_t jbase = PASS == 0 ? 0 : blockIdx.x << TB;
 		const auto seq = std::make_integer_sequence<int, G::ROUNDS>();
