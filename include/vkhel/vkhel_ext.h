@@ -136,7 +136,9 @@ int vkhel_ext_set_ntt_algo(struct vkhel_ctx *, int algo);
  * fastest per size on this context. */
 int vkhel_ext_autotune(struct vkhel_ctx *, uint32_t logn_lo, uint32_t logn_hi,
 		uint32_t batch);
-/* Tile size (log2 words) in use for log2 n, or -1 on error. */
+/* Tile size (log2 words) in use for log2 n, or -1 on error.  (Untuned,
+ * batches of n = 2^14 that fill the device run in one pass on 2^14 tiles
+ * instead of the 2^12 tiles reported.) */
 int vkhel_ext_tile_bits(struct vkhel_ctx *, uint32_t logn);
 /* tile_bits 11..14, or 0 for the built-in default. */
 int vkhel_ext_set_tile_bits(struct vkhel_ctx *, uint32_t logn, int tile_bits);

@@ -191,7 +191,8 @@ bool ntt_fused_supported(uint32_t logn) {
 }
 
 // Untuned default tile per size, from batched timings on MI355X (2^25 words
-// per batch, split passes): 2^12 tiles from n = 2^14 to 2^17, 2^13 above;
+// per batch, split passes): 2^12 tiles from n = 2^14 to 2^17 (2^14: unless
+// tile_bits_for_tasks picks one pass), 2^13 above;
 // sizes up to 2^13 run in one pass on a 2^13 tile.
 static int default_tile_bits(uint32_t logn) {
 	if (logn <= 13)
@@ -202,6 +203,30 @@ static int default_tile_bits(uint32_t logn) {
 int tile_bits_for(const vkhel_ctx *ctx, uint32_t logn) {
 	const int tb = logn < ctx->tile_bits.size() ? ctx->tile_bits[logn] : 0;
 	return tb ? tb : default_tile_bits(logn);
+}
+
+// The tile for `ntasks` transforms at once.  Untuned n = 2^14 runs in one
+// pass on 2^14-word tiles, one workgroup per CU, where that fills the CUs:
+// its time goes in steps of one CU-full of polynomials, the two passes' with
+// their number.  Forward + inverse on MI355X (256 CUs), two passes against
+// one, us: moduli below 2^50, 128 polynomials 39 / 38, 192 47 / 42, 256
+// 59 / 48, 320 73 / 77, 384 84 / 80, 512 111 / 89, 576 114 / 118, 768
+// 154 / 129, 2048 383 / 328; 60 bits, 192 55 / 54, 256 67 / 60, 320 83 / 100,
+// 384 96 / 103, 512 121 / 117, 576 133 / 154, 768 175 / 170, 1024 226 / 223,
+// 2048 426 / 433.  So: three quarters of the last step filled on average
+// over the steps for the double-precision class, seven eighths and at most
+// four steps for the others (arithmetic takes longer there, memory less).
+static int tile_bits_for_tasks(const vkhel_ctx *ctx, uint32_t logn,
+		uint32_t ntasks, int mc) {
+	if (logn == 14 && !ctx->tile_bits[logn] && !ctx->pass_mode[logn] &&
+			!ctx->split[logn] && !ctx->tile_bits2[logn] && ctx->cu_count > 0) {
+		const uint64_t cus = (uint64_t) ctx->cu_count;
+		const uint64_t steps = (ntasks + cus - 1) / cus;
+		if (mc == kClassFp ? 4 * (uint64_t) ntasks >= 3 * steps * cus
+				: 8 * (uint64_t) ntasks >= 7 * steps * cus && steps <= 4)
+			return 14;
+	}
+	return tile_bits_for(ctx, logn);
 }
 
 // Split two-pass transforms run in chunks of at most 2^25 words (256 MiB)
@@ -383,7 +408,7 @@ int launch_fused_tasks(const vkhel_ctx *ctx, const NttTask *dev_tasks,
 		return VKHEL_OK;
 	if (!fused_supported(logn))
 		return fail(VKHEL_ERR_INVALID, "fused NTT: unsupported log2 n = %u", logn);
-	const int tb = tile_bits_for(ctx, logn);
+	const int tb = tile_bits_for_tasks(ctx, logn, ntasks, mc);
 	const FusedEntry &e = fused_entry(logn, tb);
 	if (pass_mode_of(ctx, logn) == 3 && e.tiles > 1 && dev_tasks &&
 			handoff_state && handoff_bytes >= handoff_state_bytes(ntasks))
@@ -491,10 +516,10 @@ int launch_ntt(vkhel_ctx *ctx, const DevTables &t, const uint64_t *in,
 	const uint32_t logn = t.c.logn;
 	if (ctx->ntt_algo == VKHEL_NTT_RADIX2 || !fused_supported(logn))
 		return launch_radix2(t, in, out, batch, inverse, s);
+	const int mc = modulus_class(t.c.q);
 	return launch_fused_impl(ctx, make_task(t, in, out, inverse), nullptr, batch,
-			logn,
-			tile_bits_for(ctx, logn), use_split(ctx, logn), inverse,
-			modulus_class(t.c.q), s);
+			logn, tile_bits_for_tasks(ctx, logn, batch, mc), use_split(ctx, logn),
+			inverse, mc, s);
 }
 
 static void transform(const vkhel_vector *op, vkhel_vector *res,
