@@ -130,7 +130,7 @@ struct Tuning {
 	}
 
 	int run(vkhel_ctx *ctx, bool inverse) {
-		return launch_fused_tasks(ctx, tasks, polys, logn, inverse, mc,
+		return launch_fused_tasks(ctx, tasks, polys, logn, inverse, mc, false,
 				ctx->stream, state, state_bytes);
 	}
 

@@ -303,10 +303,32 @@ static std::vector<Segment> segment(std::vector<NttTask> &tasks,
 		const int mc = modulus_class(tasks[i].c.q);
 		if (segs.empty() || segs.back().logn != tasks[i].c.logn ||
 				segs.back().mc != mc)
-			segs.push_back(Segment{i, 0, tasks[i].c.logn, mc, 0, kNoHandoff});
+			segs.push_back(Segment{i, 0, tasks[i].c.logn, mc, 0, kNoHandoff, false});
 		segs.back().count++;
 	}
 	return segs;
+}
+
+// Input words from which a segment's first passes stream their input.
+constexpr uint64_t kStreamWords = 1ull << 24;
+
+// A segment whose tasks all read other memory than they write, and which
+// together with its results fills the 256 MB last-level cache, loads its
+// input with the nontemporal hint in its first pass: loaded ordinarily the
+// input, which is not read again, drives out the first pass's results before
+// the second reads them.  Forward + inverse on MI355X, us: 512 x 2^16 at 50
+// bits 394 -> 367, at 60 bits 456 -> 440, 256 x 2^16 at 50 bits 207 -> 198,
+// 1024 x 2^15 at 60 bits 438 -> 418, 256 x 2^17 483 -> 464; products of
+// 2^26 words at 55 bits 1124 -> 1112.  Smaller input may wait in the cache from
+// what wrote it, and the hint then costs (128 x 2^16 forward, input cached,
+// 47 -> 52); so it does in place (512 x 2^16 forward 175 -> 184).
+static void stream_input(std::vector<Segment> &segs,
+		const std::vector<NttTask> &tasks, uint64_t words) {
+	for (Segment &g : segs) {
+		g.stream = (uint64_t) g.count << g.logn >= words;
+		for (uint32_t i = 0; i < g.count && g.stream; i++)
+			g.stream = tasks[g.off + i].in != tasks[g.off + i].out;
+	}
 }
 
 // elemmod(a, pm, q) over n words into out (src/vector.c:342-386: the
@@ -529,6 +551,9 @@ int plan_tasks(vkhel_ctx *ctx, const Job *const *jobs, size_t njobs,
 	ts.seg_fwd2 = segment(ts.fwd2, true);
 	ts.seg_pm_col = segment(ts.pm_col, false);
 	ts.seg_pm = segment(ts.pm, false);
+	stream_input(ts.seg_fwd, ts.fwd, kStreamWords);
+	stream_input(ts.seg_inv, ts.inv, kStreamWords);
+	stream_input(ts.seg_pm_col, ts.pm_col, kStreamWords);
 	for (auto *segs : {&ts.seg_pm_col, &ts.seg_pm}) {
 		for (Segment &g : *segs)
 			g.tb = polymul_fused_tile(ctx, g.logn);
@@ -614,9 +639,11 @@ static int launch_segments(const vkhel_ctx *ctx,
 		int rc = VKHEL_OK;
 		if (ntt_fused_supported(g.logn)) {
 			rc = g.hoff == kNoHandoff
-				? launch_fused_tasks(ctx, dev + g.off, g.count, g.logn, inverse, g.mc, s)
-				: launch_fused_tasks(ctx, dev + g.off, g.count, g.logn, inverse, g.mc, s,
-						dt.handoff + g.hoff, dt.handoff_bytes - 4ull * g.hoff);
+				? launch_fused_tasks(ctx, dev + g.off, g.count, g.logn, inverse, g.mc,
+						g.stream, s)
+				: launch_fused_tasks(ctx, dev + g.off, g.count, g.logn, inverse, g.mc,
+						g.stream, s, dt.handoff + g.hoff,
+						dt.handoff_bytes - 4ull * g.hoff);
 		} else {
 			for (uint32_t i = 0; i < g.count && rc == VKHEL_OK; i++)
 				rc = launch_task_ntt(host[g.off + i], inverse, s);
@@ -656,16 +683,18 @@ static int launch_polymul_segments(const TaskSet &ts, const DeviceTasks &dt,
 		hipStream_t s) {
 	for (const Segment &g : ts.seg_pm) {
 		const NttTask *cols = nullptr;
+		bool stream = false;
 		for (const Segment &c : ts.seg_pm_col) {
 			if (c.logn == g.logn && c.mc == g.mc) {
 				if (c.count != 2 * g.count)
 					return fail(VKHEL_ERR_INVALID, "polymul plan: column segment "
 							"of %u tasks for %u products", c.count, g.count);
 				cols = dt.pm_col + c.off;
+				stream = c.stream;
 			}
 		}
 		const int rc = launch_polymul_tasks(cols, dt.pm + g.off, g.count, g.logn,
-				g.tb, g.mc, s);
+				g.tb, g.mc, stream, s);
 		if (rc != VKHEL_OK)
 			return rc;
 	}

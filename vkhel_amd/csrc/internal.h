@@ -243,11 +243,13 @@ NttTask make_task(const DevTables &t, const uint64_t *in, uint64_t *out,
 // Device-resident tasks that share log2 n (which selects the compiled
 // kernel), direction and modulus class (mc, modulus_class() of every q);
 // the context supplies the tuned tile size.
+// stream: the first of two passes loads its input with the nontemporal hint.
 // Pass mode 3 (one launch for both passes, k_ntt_handoff) needs a state
 // buffer of handoff_state_bytes(ntasks); without one the passes run split.
 int launch_fused_tasks(const vkhel_ctx *ctx, const NttTask *dev_tasks,
-		uint32_t ntasks, uint32_t logn, bool inverse, int mc, hipStream_t st,
-		uint32_t *handoff_state = nullptr, uint64_t handoff_bytes = 0);
+		uint32_t ntasks, uint32_t logn, bool inverse, int mc, bool stream,
+		hipStream_t st, uint32_t *handoff_state = nullptr,
+		uint64_t handoff_bytes = 0);
 uint64_t handoff_state_bytes(uint32_t ntasks);
 // True when transforms of log2 n run both passes in one launch on ctx
 // (pass mode 3 at a two-pass size).
@@ -271,7 +273,8 @@ int polymul_fused_tile(const vkhel_ctx *ctx, uint32_t logn);
 // b (into scratch), which the pm task then names as in and in2; one-tile
 // sizes take col_tasks null and read a and b themselves.
 int launch_polymul_tasks(const NttTask *col_tasks, const NttTask *pm_tasks,
-		uint32_t ntasks, uint32_t logn, int tile_bits, int mc, hipStream_t st);
+		uint32_t ntasks, uint32_t logn, int tile_bits, int mc, bool stream,
+		hipStream_t st);
 // One fused polynomial product without task arrays: the column tasks of a
 // and b (two-pass sizes, cols true) and the product task passed by value.
 int launch_polymul_one(const NttTask &col_a, const NttTask &col_b,

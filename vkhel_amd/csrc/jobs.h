@@ -51,6 +51,8 @@ struct Segment {
 	// word offset of this segment's state in DeviceTasks::handoff when it
 	// runs both passes in one launch (pass mode 3), else kNoHandoff
 	uint32_t hoff;
+	// first passes load their input with the nontemporal hint (stream_input)
+	bool stream;
 };
 constexpr uint32_t kNoHandoff = 0xffffffffu;
 

@@ -270,8 +270,9 @@ static PassPlan pass_plan(const vkhel_ctx *ctx, uint32_t logn, int tile_bits) {
 // kernels).
 static int launch_fused_impl(const vkhel_ctx *ctx, const NttTask &uniform,
 		const NttTask *dev_tasks, uint32_t ntasks, uint32_t logn, int tile_bits,
-		bool split, bool inverse, int mc, hipStream_t st) {
+		bool split, bool inverse, int mc, bool stream, hipStream_t st) {
 	const FusedEntry &e = fused_entry(logn, tile_bits);
+	const uint32_t first_pass = stream ? kStreamIn : 0u;
 	if (split && e.tiles > 1) {
 		const PassPlan pp = pass_plan(ctx, logn, tile_bits);
 		const FusedEntry &e1 = *pp.e1, &e2 = *pp.e2;
@@ -294,12 +295,12 @@ static int launch_fused_impl(const vkhel_ctx *ctx, const NttTask &uniform,
 			// forward: columns, then rows; inverse: rows, then columns
 			if (!inverse) {
 				hipLaunchKernelGGL(e1.k[mc].fwd_a[s], dim3(e1.tiles, count),
-						dim3(e1.threads), 0, st, u, d, 0u);
+						dim3(e1.threads), 0, st, u, d, first_pass);
 				hipLaunchKernelGGL(e2.k[mc].fwd_b[s], dim3(e2.tiles, count),
 						dim3(e2.threads), 0, st, u, d, kSecondPass | kReversed);
 			} else {
 				hipLaunchKernelGGL(e2.k[mc].inv_b[s], dim3(e2.tiles, count),
-						dim3(e2.threads), 0, st, u, d, 0u);
+						dim3(e2.threads), 0, st, u, d, first_pass);
 				hipLaunchKernelGGL(e1.k[mc].inv_a[s], dim3(e1.tiles, count),
 						dim3(e1.threads), 0, st, u, d, kSecondPass | kReversed);
 			}
@@ -402,8 +403,8 @@ static int launch_handoff(const vkhel_ctx *ctx, const FusedEntry &e,
 }
 
 int launch_fused_tasks(const vkhel_ctx *ctx, const NttTask *dev_tasks,
-		uint32_t ntasks, uint32_t logn, bool inverse, int mc, hipStream_t st,
-		uint32_t *handoff_state, uint64_t handoff_bytes) {
+		uint32_t ntasks, uint32_t logn, bool inverse, int mc, bool stream,
+		hipStream_t st, uint32_t *handoff_state, uint64_t handoff_bytes) {
 	if (ntasks == 0)
 		return VKHEL_OK;
 	if (!fused_supported(logn))
@@ -416,7 +417,7 @@ int launch_fused_tasks(const vkhel_ctx *ctx, const NttTask *dev_tasks,
 				handoff_state, st);
 	const NttTask none{};
 	return launch_fused_impl(ctx, none, dev_tasks, ntasks, logn, tb,
-			use_split(ctx, logn), inverse, mc, st);
+			use_split(ctx, logn), inverse, mc, stream, st);
 }
 
 // The context's tile when the fused product kernel exists for it (not for
@@ -441,7 +442,7 @@ int polymul_fused_tile(const vkhel_ctx *ctx, uint32_t logn) {
 static int polymul_impl(const NttTask &ucol_a, const NttTask &ucol_b,
 		const NttTask &upm, const NttTask *col_tasks, const NttTask *pm_tasks,
 		bool cols, uint32_t ntasks, uint32_t logn, int tile_bits, int mc,
-		hipStream_t st) {
+		bool stream, hipStream_t st) {
 	if (ntasks == 0)
 		return VKHEL_OK;
 	if (!fused_supported(logn))
@@ -470,7 +471,8 @@ static int polymul_impl(const NttTask &ucol_a, const NttTask &ucol_b,
 			// the forward column passes of a and b
 			if (col_tasks) {
 				hipLaunchKernelGGL(e.k[mc].fwd_a[0], dim3(e.tiles, 2 * count),
-						dim3(e.threads), 0, st, ucol_a, col_tasks + 2 * first, 0u);
+						dim3(e.threads), 0, st, ucol_a, col_tasks + 2 * first,
+						stream ? kStreamIn : 0u);
 			} else {
 				hipLaunchKernelGGL(e.k[mc].fwd_a[0], grid, dim3(e.threads), 0, st, ucol_a,
 						(const NttTask *) nullptr, 0u);
@@ -487,17 +489,18 @@ static int polymul_impl(const NttTask &ucol_a, const NttTask &ucol_b,
 }
 
 int launch_polymul_tasks(const NttTask *col_tasks, const NttTask *pm_tasks,
-		uint32_t ntasks, uint32_t logn, int tile_bits, int mc, hipStream_t st) {
+		uint32_t ntasks, uint32_t logn, int tile_bits, int mc, bool stream,
+		hipStream_t st) {
 	const NttTask none{};
 	return polymul_impl(none, none, none, col_tasks, pm_tasks,
-			col_tasks != nullptr, ntasks, logn, tile_bits, mc, st);
+			col_tasks != nullptr, ntasks, logn, tile_bits, mc, stream, st);
 }
 
 int launch_polymul_one(const NttTask &col_a, const NttTask &col_b,
 		const NttTask &pm, bool cols, uint32_t logn, int tile_bits, int mc,
 		hipStream_t st) {
 	return polymul_impl(col_a, col_b, pm, nullptr, nullptr, cols, 1, logn,
-			tile_bits, mc, st);
+			tile_bits, mc, false, st);
 }
 
 int launch_task_fused(const vkhel_ctx *ctx, const NttTask &k, bool inverse,
@@ -506,7 +509,7 @@ int launch_task_fused(const vkhel_ctx *ctx, const NttTask &k, bool inverse,
 	if (!fused_supported(logn))
 		return fail(VKHEL_ERR_INVALID, "fused NTT: unsupported log2 n = %u", logn);
 	return launch_fused_impl(ctx, k, nullptr, 1, logn, tile_bits_for(ctx, logn),
-			use_split(ctx, logn), inverse, modulus_class(k.c.q), st);
+			use_split(ctx, logn), inverse, modulus_class(k.c.q), false, st);
 }
 
 int launch_ntt(vkhel_ctx *ctx, const DevTables &t, const uint64_t *in,
@@ -519,7 +522,7 @@ int launch_ntt(vkhel_ctx *ctx, const DevTables &t, const uint64_t *in,
 	const int mc = modulus_class(t.c.q);
 	return launch_fused_impl(ctx, make_task(t, in, out, inverse), nullptr, batch,
 			logn, tile_bits_for_tasks(ctx, logn, batch, mc), use_split(ctx, logn),
-			inverse, mc, s);
+			inverse, mc, false, s);
 }
 
 static void transform(const vkhel_vector *op, vkhel_vector *res,

@@ -20,7 +20,8 @@ typedef void (*PassKernel)(NttTask, const NttTask *, uint32_t);
 // second pass of a direction.  kReversed: workgroup row y takes polynomial
 // gridDim.y - 1 - y, so that a pass starts on the polynomials the previous
 // launch wrote last, which are the ones still held in the last-level cache.
-constexpr uint32_t kSecondPass = 1, kReversed = 2;
+// kStreamIn (first passes): the input loads carry the nontemporal hint.
+constexpr uint32_t kSecondPass = 1, kReversed = 2, kStreamIn = 4;
 
 // Both passes of a two-pass size in one persistent grid (k_ntt_handoff):
 // (uniform, tasks, polynomials, state words, spin limit).
@@ -396,10 +397,9 @@ __device__ __forceinline__ uint64_t gload(const uint64_t *p, uint32_t i) {
 
 // A transform's input words, read once.  One-tile transforms load them
 // with the nontemporal hint (measured on MI355X, 2^25-word batches: 3-6%
-// faster at n = 2^10, 0-2% at 2^12 and 2^13); two-pass transforms keep
-// ordinary loads (with the hint there, 2^16 measured up to 4% slower: the
-// second pass reads the first pass's output from the last-level cache,
-// and nontemporal stores were slower still).
+// faster at n = 2^10, 0-2% at 2^12 and 2^13); two-pass transforms only where
+// the host asks for it (kStreamIn, batch.hip stream_input).  Nontemporal
+// stores of the results were slower (512 x 2^16 forward 174 -> 187 us).
 template <int PASS>
 __device__ __forceinline__ uint64_t gload_in(const uint64_t *p, uint32_t i) {
 	if constexpr (PASS == 0)
@@ -613,6 +613,13 @@ constexpr bool writes_result() {
 	return G::P == 0 || G::P == (INV ? 1 : 2);
 }
 
+// First passes that may load with the nontemporal hint on request (one-tile
+// transforms always do): those that read whole 128-byte lines.
+template <class G, bool INV>
+constexpr bool may_stream() {
+	return G::P != 0 && reads_input<G, INV>() && (G::P == 2 || G::CB >= 4);
+}
+
 template <class G, bool INV, int R>
 constexpr int round_stages() {
 	return Round<G, INV, R>::BHI - Round<G, INV, R>::BLO;
@@ -803,7 +810,7 @@ template <class G, bool INV, int R, int LOGN, bool TRAIL, int MC, int IO = 0>
 __device__ __forceinline__ void run_round(uint64_t v[8], Twiddle<MC> w[7],
 		uint32_t tp, const uint64_t *src, const uint64_t *src2, uint64_t *dst,
 		uint64_t *lds, uint32_t jbase, uint32_t gbase, const Twiddles<MC> &tw,
-		const NttConsts &c, bool final) {
+		const NttConsts &c, bool final, bool stream) {
 	using RD = Round<G, INV, R>;
 	constexpr int F = RD::F;
 	constexpr bool FIRST_ROUND = R == 0;
@@ -813,6 +820,7 @@ __device__ __forceinline__ void run_round(uint64_t v[8], Twiddle<MC> w[7],
 	constexpr bool KEEP = LAST_ROUND && (IO & kIoKeep);
 	// pass whose load flavour the first round's global loads take
 	constexpr int LP = (IO & kIoStreamIn) ? 0 : G::P;
+	constexpr bool MAY_STREAM = may_stream<G, INV>();
 	constexpr uint32_t PHYS = G::PHYS;
 	constexpr int VT = G::VT;
 	static_assert(VT == 1 || !(IO & (kIoPreloaded | kIoKeep)),
@@ -846,6 +854,17 @@ __device__ __forceinline__ void run_round(uint64_t v[8], Twiddle<MC> w[7],
 					for (int k = 0; k < 8; k++)
 						lds[Staged<G>::lds_at(t, k)] = lift_word(gload_in<LP>(src,
 								Staged<G>::global_at(t, k, jbase)), c);
+				} else if (MAY_STREAM && stream) {
+					// (opaque index and values: the compiler would merge these loads
+					// with the ordinary ones and drop the hint)
+					const uint32_t to = opaque32(t);
+					uint64_t x[8];
+#pragma unroll
+					for (int k = 0; k < 8; k++)
+						x[k] = gload_in<0>(src, Staged<G>::global_at(to, k, jbase));
+#pragma unroll
+					for (int k = 0; k < 8; k++)
+						lds[Staged<G>::lds_at(t, k)] = opaque(x[k]);
 				} else {
 #pragma unroll
 					for (int k = 0; k < 8; k++)
@@ -877,6 +896,11 @@ __device__ __forceinline__ void run_round(uint64_t v[8], Twiddle<MC> w[7],
 				for (int e = 0; e < 8; e++)
 					v[e] = lift_word(gload_in<LP>(src, g0 +
 							tile_off<G>((uint32_t) e << F)), c);
+			} else if (FIRST_ROUND && RD::DIRECT && MAY_STREAM && stream) {
+				const uint32_t g0 = opaque32(tile_addr<G>(l0, jbase));
+#pragma unroll
+				for (int e = 0; e < 8; e++)
+					v[e] = gload_in<0>(src, g0 + tile_off<G>((uint32_t) e << F));
 			} else if (FIRST_ROUND && RD::DIRECT) {
 				const uint32_t g0 = tile_addr<G>(l0, jbase);
 #pragma unroll
@@ -1093,20 +1117,21 @@ template <class G, bool INV, int LOGN, bool TRAIL, int MC, int IO, int... R>
 __device__ __forceinline__ void run_rounds_v(std::integer_sequence<int, R...>,
 		uint64_t v[8], uint32_t t, const uint64_t *src, const uint64_t *src2,
 		uint64_t *dst, uint64_t *lds, uint32_t jbase, uint32_t gbase,
-		const Twiddles<MC> &tw, const NttConsts &c, bool final) {
+		const Twiddles<MC> &tw, const NttConsts &c, bool final,
+		bool stream = false) {
 	Twiddle<MC> w[7];
 	(run_round<G, INV, R, LOGN, TRAIL, MC, IO>(v, w, t, src, src2, dst, lds,
-			jbase, gbase, tw, c, final), ...);
+			jbase, gbase, tw, c, final, stream), ...);
 }
 
 template <class G, bool INV, int LOGN, bool TRAIL, int MC, int... R>
 __device__ __forceinline__ void run_rounds(std::integer_sequence<int, R...> seq,
 		uint32_t t, const uint64_t *src, const uint64_t *src2, uint64_t *dst,
 		uint64_t *lds, uint32_t jbase, uint32_t gbase, const Twiddles<MC> &tw,
-		const NttConsts &c, bool final) {
+		const NttConsts &c, bool final, bool stream = false) {
 	uint64_t v[8];
 	run_rounds_v<G, INV, LOGN, TRAIL, MC, 0>(seq, v, t, src, src2, dst, lds,
-			jbase, gbase, tw, c, final);
+			jbase, gbase, tw, c, final, stream);
 }
 
 template <int LOGN, int PASS, int TB, bool INV, int MC>
@@ -1223,7 +1248,8 @@ __attribute__((amdgpu_waves_per_eu(pass_waves(LOGN, PASS, TB)))) void k_ntt_pass
 		run_rounds<G, INV, LOGN, false, MC>(
 				std::make_integer_sequence<int, G::ROUNDS>(), threadIdx.x,
 				second ? k.out : k.in, with_in2 ? k.in2 : nullptr, k.out, lds, jbase,
-				gbase, twiddles<MC, INV>(k.tw, 1u << LOGN), k.c, second);
+				gbase, twiddles<MC, INV>(k.tw, 1u << LOGN), k.c, second,
+				flags & kStreamIn);
 	}
 }
 
