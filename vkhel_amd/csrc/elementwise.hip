@@ -65,42 +65,66 @@ struct OpModTwo {
 	}
 };
 
+typedef unsigned long long word2 __attribute__((ext_vector_type(2)));
+
+// Loads and stores of a streaming kernel, with the nontemporal hint for NT.
+template <bool NT, class T>
+__device__ __forceinline__ T stream_load(const T *p) {
+	if constexpr (NT)
+		return __builtin_nontemporal_load(p);
+	else
+		return *p;
+}
+
+template <bool NT, class T>
+__device__ __forceinline__ void stream_store(T *p, T v) {
+	if constexpr (NT)
+		__builtin_nontemporal_store(v, p);
+	else
+		*p = v;
+}
+
 // VEC: every pointer is 16-byte aligned and two words move per access;
 // otherwise (a vector view at an odd word offset) one word per access.
-template <class Op, bool VEC>
+// NT: operands and result together exceed the last-level cache
+// (streams_past_cache).
+template <class Op, bool VEC, bool NT>
 __global__ __launch_bounds__(256) void k_binary(const uint64_t *a,
 		const uint64_t *b, uint64_t *out, uint64_t len, Op op) {
 	const uint64_t stride = (uint64_t) gridDim.x * blockDim.x;
 	uint64_t i = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
 	if constexpr (VEC) {
 		for (const uint64_t pairs = len >> 1; i < pairs; i += stride) {
-			const ulonglong2 x = ((const ulonglong2 *) a)[i];
-			const ulonglong2 y = ((const ulonglong2 *) b)[i];
-			((ulonglong2 *) out)[i] = make_ulonglong2(op(x.x, y.x), op(x.y, y.y));
+			const word2 x = stream_load<NT>((const word2 *) a + i);
+			const word2 y = stream_load<NT>((const word2 *) b + i);
+			const word2 r = {op(x.x, y.x), op(x.y, y.y)};
+			stream_store<NT>((word2 *) out + i, r);
 		}
 		if ((len & 1) && blockIdx.x == 0 && threadIdx.x == 0)
 			out[len - 1] = op(a[len - 1], b[len - 1]);
 	} else {
 		for (; i < len; i += stride)
-			out[i] = op(a[i], b[i]);
+			stream_store<NT>(out + i, op(stream_load<NT>(a + i),
+						stream_load<NT>(b + i)));
 	}
 }
 
-template <class Op, bool VEC>
+template <class Op, bool VEC, bool NT>
 __global__ __launch_bounds__(256) void k_unary(const uint64_t *a,
 		uint64_t *out, uint64_t len, Op op) {
 	const uint64_t stride = (uint64_t) gridDim.x * blockDim.x;
 	uint64_t i = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
 	if constexpr (VEC) {
 		for (const uint64_t pairs = len >> 1; i < pairs; i += stride) {
-			const ulonglong2 x = ((const ulonglong2 *) a)[i];
-			((ulonglong2 *) out)[i] = make_ulonglong2(op(x.x), op(x.y));
+			const word2 x = stream_load<NT>((const word2 *) a + i);
+			const word2 r = {op(x.x), op(x.y)};
+			stream_store<NT>((word2 *) out + i, r);
 		}
 		if ((len & 1) && blockIdx.x == 0 && threadIdx.x == 0)
 			out[len - 1] = op(a[len - 1]);
 	} else {
 		for (; i < len; i += stride)
-			out[i] = op(a[i]);
+			stream_store<NT>(out + i, op(stream_load<NT>(a + i)));
 	}
 }
 
@@ -131,17 +155,44 @@ static unsigned grid_for(uint64_t len) {
 	return (unsigned) std::max<uint64_t>(1, std::min<uint64_t>(blocks, 1u << 20));
 }
 
+// Vectors of more than 256 MB between them cannot wait in the last-level cache
+// for or after the call: their words move with the nontemporal hint.
+static bool streams_past_cache(uint64_t len, uint64_t vectors) {
+	return len * vectors * 8 > 256ull << 20;
+}
+
+// out may be a or b; every thread reads its words before it writes them.
+template <class Op, bool NT>
+static void launch_binary_as(const uint64_t *a, const uint64_t *b, uint64_t *out,
+		uint64_t len, Op op, hipStream_t s) {
+	if (aligned16(a) && aligned16(b) && aligned16(out))
+		hipLaunchKernelGGL((k_binary<Op, true, NT>), dim3(grid_for(len)), dim3(256),
+				0, s, a, b, out, len, op);
+	else
+		hipLaunchKernelGGL((k_binary<Op, false, NT>), dim3(grid_for(2 * len)),
+				dim3(256), 0, s, a, b, out, len, op);
+}
+
+template <class Op, bool NT>
+static void launch_unary_as(const uint64_t *a, uint64_t *out, uint64_t len,
+		Op op, hipStream_t s) {
+	if (aligned16(a) && aligned16(out))
+		hipLaunchKernelGGL((k_unary<Op, true, NT>), dim3(grid_for(len)), dim3(256),
+				0, s, a, out, len, op);
+	else
+		hipLaunchKernelGGL((k_unary<Op, false, NT>), dim3(grid_for(2 * len)),
+				dim3(256), 0, s, a, out, len, op);
+}
+
 template <class Op>
 int launch_binary(const uint64_t *a, const uint64_t *b, uint64_t *out,
 		uint64_t len, Op op, hipStream_t s) {
 	if (len == 0)
 		return VKHEL_OK;
-	if (aligned16(a) && aligned16(b) && aligned16(out))
-		hipLaunchKernelGGL((k_binary<Op, true>), dim3(grid_for(len)), dim3(256), 0,
-				s, a, b, out, len, op);
+	if (streams_past_cache(len, 3))
+		launch_binary_as<Op, true>(a, b, out, len, op, s);
 	else
-		hipLaunchKernelGGL((k_binary<Op, false>), dim3(grid_for(2 * len)),
-				dim3(256), 0, s, a, b, out, len, op);
+		launch_binary_as<Op, false>(a, b, out, len, op, s);
 	return hip_ok(hipGetLastError(), "launch") ? VKHEL_OK : VKHEL_ERR_DEVICE;
 }
 
@@ -150,12 +201,10 @@ int launch_unary(const uint64_t *a, uint64_t *out, uint64_t len, Op op,
 		hipStream_t s) {
 	if (len == 0)
 		return VKHEL_OK;
-	if (aligned16(a) && aligned16(out))
-		hipLaunchKernelGGL((k_unary<Op, true>), dim3(grid_for(len)), dim3(256), 0,
-				s, a, out, len, op);
+	if (streams_past_cache(len, 2))
+		launch_unary_as<Op, true>(a, out, len, op, s);
 	else
-		hipLaunchKernelGGL((k_unary<Op, false>), dim3(grid_for(2 * len)),
-				dim3(256), 0, s, a, out, len, op);
+		launch_unary_as<Op, false>(a, out, len, op, s);
 	return hip_ok(hipGetLastError(), "launch") ? VKHEL_OK : VKHEL_ERR_DEVICE;
 }
 
