@@ -425,6 +425,7 @@ int plan_tasks(vkhel_ctx *ctx, const Job *const *jobs, size_t njobs,
 					f.c.lift_add = q - ql % q;
 					f.c.scale_w = w;
 					f.c.scale_wp = shoup63_factor(w, q);
+					f.c.fscale = fp_center(w, q);
 					f.in2 = j.a->dev + off;
 					ts.fwd2.push_back(f);
 					break;

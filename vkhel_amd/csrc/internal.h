@@ -51,9 +51,9 @@ struct NttConsts {
 	// word i becomes (in2[i] - y) * scale_w mod q, scale_wp the packed
 	// Shoup companion of scale_w
 	uint64_t scale_w, scale_wp;
-	// the double-precision class (q < kFpQ): q, 1/q rounded, and ninv and w1n
-	// as centered residues (fp_center)
-	double fq, fqinv, fninv, fw1n;
+	// the double-precision class (q < kFpQ): q, 1/q rounded, and ninv, w1n
+	// and scale_w as centered residues (fp_center)
+	double fq, fqinv, fninv, fw1n, fscale;
 	uint32_t bshift;  // bits - 2
 	uint32_t logn;
 };
