@@ -206,23 +206,28 @@ int tile_bits_for(const vkhel_ctx *ctx, uint32_t logn) {
 }
 
 // The tile for `ntasks` transforms at once.  Untuned n = 2^14 runs in one
-// pass on 2^14-word tiles, one workgroup per CU, where that fills the CUs:
-// its time goes in steps of one CU-full of polynomials, the two passes' with
-// their number.  Forward + inverse on MI355X (256 CUs), two passes against
-// one, us: moduli below 2^50, 128 polynomials 39 / 38, 192 47 / 42, 256
-// 59 / 48, 320 73 / 77, 384 84 / 80, 512 111 / 89, 576 114 / 118, 768
-// 154 / 129, 2048 383 / 328; 60 bits, 192 55 / 54, 256 67 / 60, 320 83 / 100,
-// 384 96 / 103, 512 121 / 117, 576 133 / 154, 768 175 / 170, 1024 226 / 223,
-// 2048 426 / 433.  So: three quarters of the last step filled on average
-// over the steps for the double-precision class, seven eighths and at most
-// four steps for the others (arithmetic takes longer there, memory less).
+// pass on 2^14-word tiles where that fills the device: its time goes in steps
+// of one CU-full of polynomials (one workgroup per CU, or two with 32 words
+// per thread, launch_fused_impl), the two passes' with their number.  Forward
+// + inverse on MI355X (256 CUs), us, moduli below 2^50, two passes / one of
+// one workgroup per CU / one of two: 128 polynomials 39 / 41 / 43, 192
+// 48 / 42 / 46, 256 56 / 49 / 54, 320 67 / 77 / 74, 384 75 / 77 / 75, 512
+// 94 / 85 / 82, 576 106 / 111 / 104, 640 113 / 113 / 106, 768 151 / 123 / 116,
+// 1024 185 / 163 / 154, 2048 352 / 329 / 295.  At 60 bits, two passes / one:
+// 192 55 / 54, 256 67 / 60, 320 83 / 100, 384 96 / 103, 512 121 / 117, 576
+// 133 / 154, 768 175 / 170, 1024 226 / 223, 2048 426 / 433.  So: for the
+// double-precision class from three quarters of one step to a whole one, and
+// from one and a half steps on; for the others seven eighths of the last step
+// filled on average over the steps and at most four steps (arithmetic takes
+// longer there, memory less).
 static int tile_bits_for_tasks(const vkhel_ctx *ctx, uint32_t logn,
 		uint32_t ntasks, int mc) {
 	if (logn == 14 && !ctx->tile_bits[logn] && !ctx->pass_mode[logn] &&
 			!ctx->split[logn] && !ctx->tile_bits2[logn] && ctx->cu_count > 0) {
 		const uint64_t cus = (uint64_t) ctx->cu_count;
 		const uint64_t steps = (ntasks + cus - 1) / cus;
-		if (mc == kClassFp ? 4 * (uint64_t) ntasks >= 3 * steps * cus
+		if (mc == kClassFp ? (4 * (uint64_t) ntasks >= 3 * cus && steps == 1) ||
+				2 * (uint64_t) ntasks >= 3 * cus
 				: 8 * (uint64_t) ntasks >= 7 * steps * cus && steps <= 4)
 			return 14;
 	}
@@ -306,8 +311,12 @@ static int launch_fused_impl(const vkhel_ctx *ctx, const NttTask &uniform,
 			}
 		}
 	} else {
-		hipLaunchKernelGGL(inverse ? e.k[mc].inv : e.k[mc].fwd,
-				dim3(ntasks), dim3(e.threads), 0, st, uniform, dev_tasks);
+		const ClassKernels &ck = e.k[mc];
+		const bool wide = ck.wide_fwd && ntasks > (uint32_t) ctx->cu_count;
+		const FusedKernel k = wide ? (inverse ? ck.wide_inv : ck.wide_fwd)
+			: inverse ? ck.inv : ck.fwd;
+		hipLaunchKernelGGL(k, dim3(ntasks), dim3(wide ? 1 << (logn - kWideBits)
+					: e.threads), 0, st, uniform, dev_tasks);
 	}
 	return hip_ok(hipGetLastError(), "ntt fused launch") ? VKHEL_OK
 		: VKHEL_ERR_DEVICE;

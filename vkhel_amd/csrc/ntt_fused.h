@@ -34,6 +34,8 @@ typedef void (*HandoffKernel)(NttTask, const NttTask *, uint32_t, uint32_t *,
 // workgroup per tile: the default for two-pass sizes).
 struct ClassKernels {
 	FusedKernel fwd, inv;
+	// the same with 32 words per thread (ntt_wide.h; null: none)
+	FusedKernel wide_fwd, wide_inv;
 	// [split]: split 0 takes the top ntt_k1 stages in pass 1, split 1 the top
 	// alt_k1 (the same kernels as split 0 where there is none)
 	PassKernel fwd_a[2], fwd_b[2], inv_b[2], inv_a[2];
@@ -1484,6 +1486,12 @@ __attribute__((amdgpu_waves_per_eu(pm_waves(LOGN, TB)))) void k_ntt_pm(
 	}
 }
 
+}  // namespace vk
+
+#include "ntt_wide.h"
+
+namespace vk {
+
 // The pass kernels of one (size, pass, direction, tile) for both splits;
 // the alternative split is instantiated only where it exists (else it names
 // the default kernel).
@@ -1496,6 +1504,11 @@ constexpr void set_passes(PassKernel k[2]) {
 // The whole-polynomial two-pass kernels and the one-launch ones are tuning
 // modes that measured slower than the split passes at every size: moduli of
 // the double-precision class run the small class's there.
+// One-pass transforms that run with 32 words per thread (ntt_wide.h).
+constexpr bool wide_ok(int logn, int tb, int mc) {
+	return mc == kClassFp && logn == 14 && tb == 14;
+}
+
 template <int LG, int TB, int MC>
 constexpr ClassKernels class_kernels() {
 	constexpr int MC2 = MC == kClassFp ? (int) kClassSmall : MC;
@@ -1503,6 +1516,10 @@ constexpr ClassKernels class_kernels() {
 	ClassKernels k{};
 	k.fwd = k_ntt_fused<LG, false, TB, MC1>;
 	k.inv = k_ntt_fused<LG, true, TB, MC1>;
+	if constexpr (wide_ok(LG, TB, MC)) {
+		k.wide_fwd = k_ntt_wide<LG, false>;
+		k.wide_inv = k_ntt_wide<LG, true>;
+	}
 	set_passes<LG, TB, MC, 1, false>(k.fwd_a);
 	set_passes<LG, TB, MC, 2, false>(k.fwd_b);
 	set_passes<LG, TB, MC, 2, true>(k.inv_b);
