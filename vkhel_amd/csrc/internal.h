@@ -234,6 +234,10 @@ struct NttTask {
 	const ulonglong2 *tw2;
 };
 
+// Words of polynomials whose passes run one after the other before the next
+// chunk's (ntt.hip).
+constexpr uint64_t kChunkWords = 1ull << 25;
+
 // Launchers (ntt.hip).  `batch` polynomials of n words, poly p at
 // in + p*n / out + p*n, all with the same tables.  Stream-ordered.
 int launch_ntt(vkhel_ctx *ctx, const DevTables &t, const uint64_t *in,

@@ -246,8 +246,8 @@ static int tile_bits_for_tasks(const vkhel_ctx *ctx, uint32_t logn,
 // reversed chunks against 2^24 in order); 256 x 2^17 0.238 -> 0.224,
 // 32 x 2^20 0.348 -> 0.332, 1024 x 2^15 0.199 -> 0.189.  Smaller chunks add
 // launch tails (2^23-word reversed chunks: 0.236 at 512 x 2^16).  Chunks
-// also keep the grid's y dimension within its limit of 65535.
-constexpr uint64_t kChunkWords = 1ull << 25;
+// also keep the grid's y dimension within its limit of 65535.  (kChunkWords,
+// internal.h)
 
 // The kernels of a two-pass size on a context: pass 1 (columns) from the
 // tile_bits table, pass 2 (rows) from the tile_bits2 one, both with the
