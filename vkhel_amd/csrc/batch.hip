@@ -360,6 +360,97 @@ static void order_pointwise(std::vector<PointTask> &h) {
 			const PointTask &y) { return x.len > y.len; });
 }
 
+// True when the steps of a task set may run in any order and side by side:
+// every job is done by one step (two-phase jobs leave tasks in `post` or
+// `fwd2`, or products without a fused kernel), none writes words that another
+// reads or writes, and none hands over between workgroups in one launch.
+static bool steps_independent(const vkhel_ctx *ctx, const Job *const *jobs,
+		size_t njobs, const TaskSet &ts) {
+	if (!ts.post.empty() || !ts.fwd2.empty() || !ts.post2.empty() ||
+			ts.handoff_words)
+		return false;
+	struct Range {
+		uintptr_t lo, hi;
+		uint32_t job;
+		bool write;
+	};
+	std::vector<Range> ranges;
+	ranges.reserve(3 * njobs);
+	for (uint32_t i = 0; i < njobs; i++) {
+		const Job &j = *jobs[i];
+		const uint64_t n = j.tables[0]->n, bytes = 8 * n * j.tables.size();
+		if (j.op == VKHEL_JOB_POLYMUL &&
+				!polymul_fused_tile(ctx, (uint32_t) (bitlen(n) - 1)))
+			return false;
+		const auto add = [&](const vkhel_vector *v, bool write) {
+			const uintptr_t lo = (uintptr_t) v->dev;
+			ranges.push_back(Range{lo, lo + bytes, i, write});
+		};
+		add(j.a, false);
+		if (j.b)
+			add(j.b, false);
+		add(j.res, true);
+	}
+	std::sort(ranges.begin(), ranges.end(), [](const Range &x, const Range &y) {
+		return x.lo < y.lo;
+	});
+	// the two furthest ends so far of different jobs, over all ranges and over
+	// the written ones
+	struct Ends {
+		uintptr_t end[2] = {0, 0};
+		uint32_t job[2] = {~0u, ~0u};
+		void put(uintptr_t e, uint32_t j) {
+			if (j == job[0]) {
+				end[0] = std::max(end[0], e);
+			} else if (e > end[0]) {
+				end[1] = end[0];
+				job[1] = job[0];
+				end[0] = e;
+				job[0] = j;
+			} else if (e > end[1]) {
+				end[1] = e;
+				job[1] = j;
+			}
+		}
+		uintptr_t other(uint32_t j) const {
+			return end[j == job[0] ? 1 : 0];
+		}
+	} all, written;
+	for (const Range &r : ranges) {
+		if ((r.write ? all : written).other(r.job) > r.lo)
+			return false;
+		all.put(r.hi, r.job);
+		if (r.write)
+			written.put(r.hi, r.job);
+	}
+	return true;
+}
+
+// Batches of at most this many kernel launches are enqueued directly on
+// each launch: a graph replay costs about 10 us more on the device than
+// the same launches from the host stream (measured on MI355X: 512 x 2^16
+// forward transforms, two launches, 0.231 ms replayed against 0.214 ms
+// enqueued; 8192 x 2^12, one launch, 0.148 against 0.137), while batches
+// of many launches (a 1000-job mixed batch, about 50) time the same either
+// way and keep the graph for its lower host cost.
+constexpr size_t kDirectLaunchMax = 8;
+
+// True when a task set's steps would run otherwise if they were independent:
+// with segments of both directions to run beside each other, or launches
+// enough for a graph (kDirectLaunchMax).  (Sorting the words of 4096 jobs takes
+// a fifth as long as planning them.)
+static bool order_matters(const vkhel_ctx *ctx, const TaskSet &ts) {
+	if (2 * (ts.seg_fwd.size() + ts.seg_inv.size()) + 3 * ts.seg_pm.size() +
+			4 * !ts.pt.empty() > kDirectLaunchMax)
+		return true;
+	for (const Segment &f : ts.seg_fwd)
+		for (const Segment &i : ts.seg_inv)
+			if (f.logn == i.logn && f.mc == i.mc &&
+					launch_both_ok(ctx, f.count, i.count, f.logn, f.mc))
+				return true;
+	return false;
+}
+
 int plan_tasks(vkhel_ctx *ctx, const Job *const *jobs, size_t njobs,
 		uint64_t *scratch, TaskSet &ts) {
 	ts = TaskSet();
@@ -571,6 +662,8 @@ int plan_tasks(vkhel_ctx *ctx, const Job *const *jobs, size_t njobs,
 			}
 		}
 	}
+	ts.independent = order_matters(ctx, ts) &&
+		steps_independent(ctx, jobs, njobs, ts);
 	return VKHEL_OK;
 }
 
@@ -694,13 +787,16 @@ static int launch_polymul_segment(const TaskSet &ts, const DeviceTasks &dt,
 // One step of a task set: a segment's transforms or products, or a phase of
 // pointwise tasks (segment null).
 struct Step {
-	enum Kind { kFwd, kProducts, kPoint, kInv, kPost, kFwd2, kPost2 } kind;
+	enum Kind { kFwd, kProducts, kPoint, kInv, kPost, kFwd2, kPost2, kBoth,
+		kNone } kind;
 	const Segment *seg;
 	uint64_t words;  // moved by its launches, roughly
+	const Segment *inv = nullptr;  // kBoth: the inverse segment beside seg
 };
 
-// The steps in the order the phases run them.
-static std::vector<Step> steps_of(const TaskSet &ts) {
+// The steps in the order the phases run them; independent steps of both
+// directions of one size and class together where launch_both_ok.
+static std::vector<Step> steps_of(const vkhel_ctx *ctx, const TaskSet &ts) {
 	std::vector<Step> steps;
 	const auto segments = [&](Step::Kind kind, const std::vector<Segment> &segs,
 			uint64_t passes, int tile) {
@@ -722,6 +818,26 @@ static std::vector<Step> steps_of(const TaskSet &ts) {
 	points(Step::kPost, ts.post);
 	segments(Step::kFwd2, ts.seg_fwd2, 2, 13);
 	points(Step::kPost2, ts.post2);
+	if (!ts.independent)
+		return steps;
+	for (Step &f : steps) {
+		if (f.kind != Step::kFwd)
+			continue;
+		const auto i = std::find_if(steps.begin(), steps.end(), [&](const Step &x) {
+			return x.kind == Step::kInv && x.seg->logn == f.seg->logn &&
+				x.seg->mc == f.seg->mc;
+		});
+		if (i != steps.end() && launch_both_ok(ctx, f.seg->count, i->seg->count,
+					f.seg->logn, f.seg->mc)) {
+			f.kind = Step::kBoth;
+			f.inv = i->seg;
+			f.words += i->words;
+			i->kind = Step::kNone;
+		}
+	}
+	steps.erase(std::remove_if(steps.begin(), steps.end(), [](const Step &x) {
+		return x.kind == Step::kNone;
+	}), steps.end());
 	return steps;
 }
 
@@ -730,6 +846,9 @@ static int enqueue_step(const vkhel_ctx *ctx, const TaskSet &ts,
 	switch (st.kind) {
 	case Step::kFwd:
 		return launch_segment(ctx, *st.seg, ts.fwd, dt.fwd, false, dt, s);
+	case Step::kBoth:
+		return launch_both_tasks(ctx, dt.fwd + st.seg->off, st.seg->count,
+				dt.inv + st.inv->off, st.inv->count, st.seg->logn, st.seg->mc, s);
 	case Step::kProducts:
 		return launch_polymul_segment(ts, dt, *st.seg, s);
 	case Step::kPoint:
@@ -747,85 +866,12 @@ static int enqueue_step(const vkhel_ctx *ctx, const TaskSet &ts,
 
 int enqueue_tasks(const vkhel_ctx *ctx, const TaskSet &ts,
 		const DeviceTasks &dt, hipStream_t s) {
-	for (const Step &st : steps_of(ts)) {
+	for (const Step &st : steps_of(ctx, ts)) {
 		const int rc = enqueue_step(ctx, ts, dt, st, s);
 		if (rc != VKHEL_OK)
 			return rc;
 	}
 	return VKHEL_OK;
-}
-
-// True when the steps of a task set may run in any order and side by side:
-// every job is done by one step (two-phase jobs leave tasks in `post` or
-// `fwd2`, or products without a fused kernel), none writes words that another
-// reads or writes, and no segment takes more than one chunk (those fill the
-// device, and beside each other lose what their second passes find cached:
-// 2048 x 2^16 forward and inverse at 60 bits 1722 us in order, 1773 in
-// branches) or hands over between workgroups in one launch.
-static bool steps_independent(const vkhel_ctx *ctx, const std::vector<Job> &jobs,
-		const TaskSet &ts) {
-	if (!ts.post.empty() || !ts.fwd2.empty() || !ts.post2.empty() ||
-			ts.handoff_words)
-		return false;
-	for (const auto *segs : {&ts.seg_fwd, &ts.seg_pm, &ts.seg_inv})
-		for (const Segment &g : *segs)
-			if (((uint64_t) g.count << g.logn) > kChunkWords)
-				return false;
-	struct Range {
-		uintptr_t lo, hi;
-		uint32_t job;
-		bool write;
-	};
-	std::vector<Range> ranges;
-	ranges.reserve(3 * jobs.size());
-	for (uint32_t i = 0; i < jobs.size(); i++) {
-		const Job &j = jobs[i];
-		const uint64_t n = j.tables[0]->n, bytes = 8 * n * j.tables.size();
-		if (j.op == VKHEL_JOB_POLYMUL &&
-				!polymul_fused_tile(ctx, (uint32_t) (bitlen(n) - 1)))
-			return false;
-		const auto add = [&](const vkhel_vector *v, bool write) {
-			const uintptr_t lo = (uintptr_t) v->dev;
-			ranges.push_back(Range{lo, lo + bytes, i, write});
-		};
-		add(j.a, false);
-		if (j.b)
-			add(j.b, false);
-		add(j.res, true);
-	}
-	std::sort(ranges.begin(), ranges.end(), [](const Range &x, const Range &y) {
-		return x.lo < y.lo;
-	});
-	// the two furthest ends so far of different jobs, over all ranges and over
-	// the written ones
-	struct Ends {
-		uintptr_t end[2] = {0, 0};
-		uint32_t job[2] = {~0u, ~0u};
-		void put(uintptr_t e, uint32_t j) {
-			if (j == job[0]) {
-				end[0] = std::max(end[0], e);
-			} else if (e > end[0]) {
-				end[1] = end[0];
-				job[1] = job[0];
-				end[0] = e;
-				job[0] = j;
-			} else if (e > end[1]) {
-				end[1] = e;
-				job[1] = j;
-			}
-		}
-		uintptr_t other(uint32_t j) const {
-			return end[j == job[0] ? 1 : 0];
-		}
-	} all, written;
-	for (const Range &r : ranges) {
-		if ((r.write ? all : written).other(r.job) > r.lo)
-			return false;
-		all.put(r.hi, r.job);
-		if (r.write)
-			written.put(r.hi, r.job);
-	}
-	return true;
 }
 
 // Captures the steps of an independent task set on `s` as parallel branches:
@@ -837,12 +883,23 @@ static bool steps_independent(const vkhel_ctx *ctx, const std::vector<Job> &jobs
 // 1145 -> 890 (two branches 963, three 913, six 931), 60 jobs 520 -> 313, 16
 // jobs 107 -> 95.
 constexpr size_t kBranches = 4;
+// Segments of more than one chunk fill the device, and beside each other lose
+// what their second passes find cached (2048 x 2^16 forward and inverse at 60
+// bits 1722 us in order, 1773 in branches): such batches keep their order.
+static bool branches_pay(const TaskSet &ts) {
+	bool pay = ts.independent;
+	for (const auto *segs : {&ts.seg_fwd, &ts.seg_pm, &ts.seg_inv})
+		for (const Segment &g : *segs)
+			pay = pay && ((uint64_t) g.count << g.logn) <= kChunkWords;
+	return pay;
+}
+
 // A launch's share of its step's time, in the same unit.
 constexpr uint64_t kStepWords = 1 << 20;
 
 static int capture_branches(const vkhel_ctx *ctx, const TaskSet &ts,
 		const DeviceTasks &dt, hipStream_t s) {
-	std::vector<Step> steps = steps_of(ts);
+	std::vector<Step> steps = steps_of(ctx, ts);
 	std::stable_sort(steps.begin(), steps.end(), [](const Step &x, const Step &y) {
 		return x.words > y.words;
 	});
@@ -913,15 +970,6 @@ static void release_graph(vkhel_batch *b) {
 	b->direct = false;
 }
 
-// Batches of at most this many kernel launches are enqueued directly on
-// each launch: a graph replay costs about 10 us more on the device than
-// the same launches from the host stream (measured on MI355X: 512 x 2^16
-// forward transforms, two launches, 0.231 ms replayed against 0.214 ms
-// enqueued; 8192 x 2^12, one launch, 0.148 against 0.137), while batches
-// of many launches (a 1000-job mixed batch, about 50) time the same either
-// way and keep the graph for its lower host cost.
-constexpr size_t kDirectLaunchMax = 8;
-
 // Waits for the batch's last launch (its buffers and graph are then free
 // to change).
 static int wait_launched(vkhel_batch *b) {
@@ -973,7 +1021,7 @@ static int build(vkhel_batch *b) {
 	if (!hip_ok(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal),
 				"begin capture"))
 		return vkhel_ext_last_error();
-	rc = steps_independent(ctx, b->jobs, b->ts)
+	rc = branches_pay(b->ts)
 		? capture_branches(ctx, b->ts, b->dt, s)
 		: enqueue_tasks(ctx, b->ts, b->dt, s);
 	hipGraph_t g = nullptr;

@@ -254,6 +254,12 @@ int launch_fused_tasks(const vkhel_ctx *ctx, const NttTask *dev_tasks,
 		uint32_t ntasks, uint32_t logn, bool inverse, int mc, bool stream,
 		hipStream_t st, uint32_t *handoff_state = nullptr,
 		uint64_t handoff_bytes = 0);
+// Forward and inverse tasks of one size and class, independent of each other,
+// in launches of both directions; launch_both_ok: where that is done.
+bool launch_both_ok(const vkhel_ctx *ctx, uint32_t nfwd, uint32_t ninv,
+		uint32_t logn, int mc);
+int launch_both_tasks(const vkhel_ctx *ctx, const NttTask *fwd, uint32_t nfwd,
+		const NttTask *inv, uint32_t ninv, uint32_t logn, int mc, hipStream_t st);
 uint64_t handoff_state_bytes(uint32_t ntasks);
 // True when transforms of log2 n run both passes in one launch on ctx
 // (pass mode 3 at a two-pass size).

@@ -70,6 +70,8 @@ struct TaskSet {
 	std::vector<Segment> seg_fwd2;
 	std::vector<PointTask> post2;
 	uint64_t handoff_words = 0;  // state words of all one-launch segments
+	// the steps may run in any order and side by side (steps_independent)
+	bool independent = false;
 };
 
 // Device copies of a TaskSet's arrays, grown on demand.

@@ -429,6 +429,45 @@ int launch_fused_tasks(const vkhel_ctx *ctx, const NttTask *dev_tasks,
 			use_split(ctx, logn), inverse, mc, stream, st);
 }
 
+// Both directions in one launch: where they fit on the device at once
+// (a CU's waves hold 2^14 words), half of that for one-tile sizes.  Forward +
+// inverse on MI355X (256 CUs), in order / beside each other, us, polynomials
+// each way: 2^10 x 8 11.3 / 7.8, 2^12 x 64 16.4 / 12.4, 2^12 x 256 19.4 / 19.5,
+// 2^12 x 1024 52 / 57, 2^13 x 16 24.8 / 17.8, 2^13 x 128 28.7 / 21.4; 2^14 x 32
+// 27.5 / 20.1, 2^15 x 64 47 / 38, 2^16 x 4 27 / 17, 2^16 x 64 72 / 70, 2^16 x
+// 256 at 50 bits 192 / 214, 2^18 x 8 57 / 49, 2^18 x 32 135 / 152.  Full
+// devices lose by two directions' code and tables in their caches.
+bool launch_both_ok(const vkhel_ctx *ctx, uint32_t nfwd, uint32_t ninv,
+		uint32_t logn, int mc) {
+	if (!fused_supported(logn) || pass_mode_of(ctx, logn) || ctx->split[logn] ||
+			ctx->tile_bits2[logn])
+		return false;
+	const int tb = tile_bits_for(ctx, logn);
+	const FusedEntry &e = fused_entry(logn, tb);
+	const ClassKernels &k = e.k[mc];
+	const uint64_t room = (uint64_t) ctx->cu_count << (e.tiles == 1 ? 13 : 14);
+	return (e.tiles == 1 ? k.both : k.both_a) &&
+		((uint64_t) nfwd + ninv) << logn <= room &&
+		tile_bits_for_tasks(ctx, logn, nfwd, mc) == tb &&
+		tile_bits_for_tasks(ctx, logn, ninv, mc) == tb;
+}
+
+int launch_both_tasks(const vkhel_ctx *ctx, const NttTask *fwd, uint32_t nfwd,
+		const NttTask *inv, uint32_t ninv, uint32_t logn, int mc, hipStream_t st) {
+	const FusedEntry &e = fused_entry(logn, tile_bits_for(ctx, logn));
+	const ClassKernels &k = e.k[mc];
+	if (e.tiles == 1) {
+		hipLaunchKernelGGL(k.both, dim3(nfwd + ninv), dim3(e.threads), 0, st, fwd,
+				nfwd, inv);
+	} else {
+		const dim3 grid(e.tiles, nfwd + ninv);
+		hipLaunchKernelGGL(k.both_a, grid, dim3(e.threads), 0, st, fwd, nfwd, inv);
+		hipLaunchKernelGGL(k.both_b, grid, dim3(e.threads), 0, st, fwd, nfwd, inv);
+	}
+	return hip_ok(hipGetLastError(), "ntt fused launch") ? VKHEL_OK
+		: VKHEL_ERR_DEVICE;
+}
+
 // The context's tile when the fused product kernel exists for it (not for
 // 2^14-word tiles, whose threads each run two groups of words), else the
 // largest tile where it does.
