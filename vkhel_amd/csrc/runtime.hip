@@ -9,6 +9,7 @@
 #include <set>
 #include <vector>
 
+#include "call_wait.h"
 #include "internal.h"
 #include "numbers.h"
 
@@ -127,29 +128,35 @@ constexpr uint64_t kCallSpinWords = 1ull << 22;
 constexpr std::chrono::microseconds kCallSpin(200);
 
 int wait_call(vkhel_ctx *ctx, uint64_t words) {
-	if (words <= kCallSpinWords) {
-		uint64_t number;
-		{
-			// a number is taken and its kernel enqueued in one step, so the
-			// word only grows and passing a number means its call is done
-			std::lock_guard<std::mutex> g(ctx->done_mu);
-			number = ++ctx->done_next;
-			hipLaunchKernelGGL(k_call_done, dim3(1), dim3(1), 0, ctx->stream,
-					ctx->done, number);
-			if (!hip_ok(hipGetLastError(), "launch"))
-				return vkhel_ext_last_error();
+	uint64_t number = 0;
+	std::chrono::steady_clock::time_point until;
+	return watch_or_block([&] {
+		if (words > kCallSpinWords)
+			return false;
+		// a number is taken and its kernel enqueued in one step, so the
+		// word only grows and passing a number means its call is done
+		std::lock_guard<std::mutex> g(ctx->done_mu);
+		number = ++ctx->done_next;
+		hipLaunchKernelGGL(k_call_done, dim3(1), dim3(1), 0, ctx->stream,
+				ctx->done, number);
+		// (not launched: an error that ends the call is block()'s to report)
+		if (hipGetLastError() != hipSuccess)
+			return false;
+		until = std::chrono::steady_clock::now() + kCallSpin;
+		return true;
+	}, [&] {
+		for (int i = 0; i < 64; i++) {
+			if (__atomic_load_n(ctx->done, __ATOMIC_ACQUIRE) >= number)
+				return true;
+			__builtin_ia32_pause();
 		}
-		const auto until = std::chrono::steady_clock::now() + kCallSpin;
-		do {
-			for (int i = 0; i < 64; i++) {
-				if (__atomic_load_n(ctx->done, __ATOMIC_ACQUIRE) >= number)
-					return VKHEL_OK;
-				__builtin_ia32_pause();
-			}
-		} while (std::chrono::steady_clock::now() < until);
-	}
-	return hip_ok(hipStreamSynchronize(ctx->stream), "sync") ? VKHEL_OK
-		: vkhel_ext_last_error();
+		return false;
+	}, [&] {
+		return std::chrono::steady_clock::now() < until;
+	}, [&] {
+		return hip_ok(hipStreamSynchronize(ctx->stream), "sync") ? (int) VKHEL_OK
+			: vkhel_ext_last_error();
+	});
 }
 
 }  // namespace vk
