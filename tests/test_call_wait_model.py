@@ -1,7 +1,9 @@
 """CPU model of the end of a synchronous call (vkhel_amd/csrc/call_wait.h):
 tests/c/call_wait_model.cpp runs the library's own wait with a stand-in for
 the device.  A call returns only after its work is done, also where the
-kernel that marks its completion could not be launched."""
+kernel that marks its completion could not be launched, and it watches that
+kernel's word only in a run of calls that the program does not follow by
+synchronising the device."""
 import os
 import subprocess
 

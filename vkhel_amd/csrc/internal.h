@@ -12,6 +12,7 @@
 
 #include "vkhel/vkhel.h"
 #include "vkhel/vkhel_ext.h"
+#include "call_wait.h"
 
 namespace vk {
 
@@ -120,6 +121,7 @@ struct vkhel_ctx {
 	uint64_t *done = nullptr;
 	std::mutex done_mu;  // orders numbers as the stream sees them
 	uint64_t done_next = 0;
+	vk::CallRun call_run;  // under done_mu too
 
 	std::mutex mu;  // guards `tables` (batch and serve threads share it)
 	std::unordered_map<uint64_t, vk::DevTables *> tables;

@@ -9,7 +9,6 @@
 #include <set>
 #include <vector>
 
-#include "call_wait.h"
 #include "internal.h"
 #include "numbers.h"
 
@@ -117,25 +116,30 @@ __global__ void k_call_done(uint64_t *done, uint64_t number) {
 	__hip_atomic_store(done, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Calls of up to 2^22 words (tens of microseconds at most) wait by watching
-// a word that a one-thread kernel behind their work writes: an 8-word elemmul
-// then takes 9.0 us against 11.2 with hipStreamSynchronize, whose barrier
-// packet, completion signal and wake-up it does without (a call of two
-// launches 11.5 against 14.1).  Longer calls, and any that take over kCallSpin,
-// block in the runtime: the difference no longer shows, and a wait there
-// reports errors and yields the CPU.
+// Calls of up to 2^22 words (tens of microseconds at most) in a run of calls
+// (CallRun) wait by watching a word that a one-thread kernel behind their work
+// writes: an 8-word elemmul then takes 9.0 us against 11.2 with
+// hipStreamSynchronize, whose barrier packet, completion signal and wake-up it
+// does without (a call of two launches 11.5 against 14.1).  Longer calls, and
+// any that take over kCallSpin, block in the runtime: the difference no longer
+// shows, and a wait there reports errors and yields the CPU.
 constexpr uint64_t kCallSpinWords = 1ull << 22;
 constexpr std::chrono::microseconds kCallSpin(200);
+
+static int64_t now_ns() {
+	return std::chrono::duration_cast<std::chrono::nanoseconds>(
+			std::chrono::steady_clock::now().time_since_epoch()).count();
+}
 
 int wait_call(vkhel_ctx *ctx, uint64_t words) {
 	uint64_t number = 0;
 	std::chrono::steady_clock::time_point until;
-	return watch_or_block([&] {
-		if (words > kCallSpinWords)
-			return false;
+	const int rc = watch_or_block([&] {
 		// a number is taken and its kernel enqueued in one step, so the
 		// word only grows and passing a number means its call is done
 		std::lock_guard<std::mutex> g(ctx->done_mu);
+		if (!ctx->call_run.watch(now_ns()) || words > kCallSpinWords)
+			return false;
 		number = ++ctx->done_next;
 		hipLaunchKernelGGL(k_call_done, dim3(1), dim3(1), 0, ctx->stream,
 				ctx->done, number);
@@ -157,6 +161,9 @@ int wait_call(vkhel_ctx *ctx, uint64_t words) {
 		return hip_ok(hipStreamSynchronize(ctx->stream), "sync") ? (int) VKHEL_OK
 			: vkhel_ext_last_error();
 	});
+	std::lock_guard<std::mutex> g(ctx->done_mu);
+	ctx->call_run.end(now_ns());
+	return rc;
 }
 
 }  // namespace vk
