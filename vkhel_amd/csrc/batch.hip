@@ -548,7 +548,7 @@ int plan_tasks(vkhel_ctx *ctx, const Job *const *jobs, size_t njobs,
 				inv.c.post_p = pm;
 				if (pm != 2) {
 					inv.c.post_mu = barrett_mu(pm);
-					inv.c.post_shift = (uint32_t) (bitlen(pm) - 2);
+					inv.c.post_shift = bitlen(pm) - 2;
 				}
 				ts.inv.push_back(inv);
 				break;

@@ -211,10 +211,11 @@ __device__ __forceinline__ uint64_t post_center(uint64_t x,
 		const uint64_t u = x & 1;
 		return x > half ? 1 - u : u;
 	}
-	const uint64_t r = barrett64(x, c.post_p, c.post_mu, c.post_shift);
+	const uint64_t r = barrett64(x, c.post_p, c.post_mu,
+			(uint32_t) c.post_shift);
 	if (x > half)
 		return csub(r + c.post_p - barrett64(c.q, c.post_p, c.post_mu,
-				c.post_shift), c.post_p);
+				(uint32_t) c.post_shift), c.post_p);
 	return r;
 }
 
