@@ -261,6 +261,11 @@ int vkhel_batch_query(struct vkhel_batch *);
 /* vkhel_batch_launch + vkhel_batch_wait. */
 int vkhel_batch_run(struct vkhel_batch *);
 uint64_t vkhel_batch_num_jobs(const struct vkhel_batch *);
+/* How the batch runs as last built (0 and 0 before its first launch): its
+ * kernel launches, and how many of them start it: 1 when they follow each
+ * other, more when they run as parallel branches. */
+int vkhel_batch_shape(const struct vkhel_batch *, uint32_t *launches,
+		uint32_t *branches);
 
 /* ---- serving engine ----
  * Continuous batching over device-resident operands.  Requests use the

@@ -948,6 +948,9 @@ struct vkhel_batch {
 	// Few launches: enqueued directly on every launch instead of replaying
 	// the graph (kDirectLaunchMax).
 	bool direct = false;
+	// Of the launch sequence as built: its launches, and those that wait for
+	// no other.
+	uint32_t launches = 0, branches = 0;
 	// Private stream the batch uploads its task arrays on and captures its
 	// graph from, so that building a batch never captures work other
 	// threads enqueue on the context stream.
@@ -1030,11 +1033,14 @@ static int build(vkhel_batch *b) {
 			(void) hipGraphDestroy(g);
 		return rc != VKHEL_OK ? rc : vkhel_ext_last_error();
 	}
-	size_t nodes = 0;
-	if (!hip_ok(hipGraphGetNodes(g, nullptr, &nodes), "graph nodes")) {
+	size_t nodes = 0, roots = 0;
+	if (!hip_ok(hipGraphGetNodes(g, nullptr, &nodes), "graph nodes") ||
+			!hip_ok(hipGraphGetRootNodes(g, nullptr, &roots), "graph nodes")) {
 		(void) hipGraphDestroy(g);
 		return vkhel_ext_last_error();
 	}
+	b->launches = (uint32_t) nodes;
+	b->branches = (uint32_t) (nodes <= kDirectLaunchMax ? nodes > 0 : roots);
 	if (nodes <= kDirectLaunchMax) {
 		(void) hipGraphDestroy(g);
 		b->direct = true;
@@ -1082,6 +1088,15 @@ void vkhel_batch_clear(struct vkhel_batch *b) {
 		return;
 	b->jobs.clear();
 	b->dirty = true;
+}
+
+int vkhel_batch_shape(const struct vkhel_batch *b, uint32_t *launches,
+		uint32_t *branches) {
+	if (!b || !launches || !branches)
+		return fail(VKHEL_ERR_INVALID, "batch_shape: null argument");
+	*launches = b->launches;
+	*branches = b->branches;
+	return VKHEL_OK;
 }
 
 uint64_t vkhel_batch_num_jobs(const struct vkhel_batch *b) {

@@ -406,6 +406,13 @@ class Batch:
     def __len__(self):
         return int(_L().vkhel_batch_num_jobs(self._h))
 
+    def shape(self):
+        """vkhel_batch_shape: (kernel launches, parallel branches) of the
+        batch as last built."""
+        n, k = ctypes.c_uint32(), ctypes.c_uint32()
+        _lib.check(_L().vkhel_batch_shape(self._h, ctypes.byref(n), ctypes.byref(k)))
+        return n.value, k.value
+
     def close(self):
         if self._h:
             _L().vkhel_batch_destroy(self._h)
