@@ -79,3 +79,14 @@ def test_both_directions_together(ctx, bits, logn, nfwd, ninv, launches):
 def test_one_pass_rule(ctx, bits, polys, launches):
     assert _transforms(ctx, 14, bits, polys, 0) == (launches, 1)
     assert _transforms(ctx, 14, bits, 0, polys) == (launches, 1)
+
+
+def test_pass_mode_2_is_the_default(ctx):
+    """Mode 2 (what the tuner names) launches what mode 0 does; mode 1 runs
+    whole polynomials, both directions apart."""
+    for mode, want in ((0, [1, 1, 2, 1]), (2, [1, 1, 2, 1]), (1, [2, 2, 2, 1])):
+        got = []
+        for logn, nfwd, ninv in ((10, 8, 8), (13, 16, 16), (16, 8, 8), (14, 256, 0)):
+            ctx.set_pass_mode(logn, mode)
+            got.append(_transforms(ctx, logn, 50, nfwd, ninv)[0])
+        assert got == want, (mode, got)

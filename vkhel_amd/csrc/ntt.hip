@@ -205,6 +205,24 @@ int tile_bits_for(const vkhel_ctx *ctx, uint32_t logn) {
 	return tb ? tb : default_tile_bits(logn);
 }
 
+// Two-pass sizes run their passes as separate grids (one workgroup per tile)
+// unless tuned otherwise: at every size and batch measured, the split grids'
+// smaller register footprint and full-chip occupancy beat one workgroup per
+// polynomial.
+static int pass_mode_of(const vkhel_ctx *ctx, uint32_t logn) {
+	return logn < ctx->pass_mode.size() ? ctx->pass_mode[logn] : 0;
+}
+
+static bool use_split(const vkhel_ctx *ctx, uint32_t logn) {
+	return pass_mode_of(ctx, logn) != 1;
+}
+
+// True when a size runs its passes as the built-in choice does: pass mode 2,
+// which the tuner sets, names what mode 0 is.
+static bool default_passes(const vkhel_ctx *ctx, uint32_t logn) {
+	return pass_mode_of(ctx, logn) == 0 || pass_mode_of(ctx, logn) == 2;
+}
+
 // The tile for `ntasks` transforms at once.  Untuned n = 2^14 runs in one
 // pass on 2^14-word tiles where that fills the device: its time goes in steps
 // of one CU-full of polynomials (one workgroup per CU, or two with 32 words
@@ -222,7 +240,7 @@ int tile_bits_for(const vkhel_ctx *ctx, uint32_t logn) {
 // longer there, memory less).
 static int tile_bits_for_tasks(const vkhel_ctx *ctx, uint32_t logn,
 		uint32_t ntasks, int mc) {
-	if (logn == 14 && !ctx->tile_bits[logn] && !ctx->pass_mode[logn] &&
+	if (logn == 14 && !ctx->tile_bits[logn] && default_passes(ctx, logn) &&
 			!ctx->split[logn] && !ctx->tile_bits2[logn] && ctx->cu_count > 0) {
 		const uint64_t cus = (uint64_t) ctx->cu_count;
 		const uint64_t steps = (ntasks + cus - 1) / cus;
@@ -320,18 +338,6 @@ static int launch_fused_impl(const vkhel_ctx *ctx, const NttTask &uniform,
 	}
 	return hip_ok(hipGetLastError(), "ntt fused launch") ? VKHEL_OK
 		: VKHEL_ERR_DEVICE;
-}
-
-// Two-pass sizes run their passes as separate grids (one workgroup per tile)
-// unless tuned otherwise: at every size and batch measured, the split grids'
-// smaller register footprint and full-chip occupancy beat one workgroup per
-// polynomial.
-static int pass_mode_of(const vkhel_ctx *ctx, uint32_t logn) {
-	return logn < ctx->pass_mode.size() ? ctx->pass_mode[logn] : 0;
-}
-
-static bool use_split(const vkhel_ctx *ctx, uint32_t logn) {
-	return pass_mode_of(ctx, logn) != 1;
 }
 
 // Zeroes the state words of a one-launch two-pass transform: a kernel, not
@@ -439,8 +445,8 @@ int launch_fused_tasks(const vkhel_ctx *ctx, const NttTask *dev_tasks,
 // devices lose by two directions' code and tables in their caches.
 bool launch_both_ok(const vkhel_ctx *ctx, uint32_t nfwd, uint32_t ninv,
 		uint32_t logn, int mc) {
-	if (!fused_supported(logn) || pass_mode_of(ctx, logn) || ctx->split[logn] ||
-			ctx->tile_bits2[logn])
+	if (!fused_supported(logn) || !default_passes(ctx, logn) ||
+			ctx->split[logn] || ctx->tile_bits2[logn])
 		return false;
 	const int tb = tile_bits_for(ctx, logn);
 	const FusedEntry &e = fused_entry(logn, tb);
