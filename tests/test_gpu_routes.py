@@ -90,3 +90,17 @@ def test_pass_mode_2_is_the_default(ctx):
             ctx.set_pass_mode(logn, mode)
             got.append(_transforms(ctx, logn, 50, nfwd, ninv)[0])
         assert got == want, (mode, got)
+
+
+def test_tuned_contexts_go_by_number_and_class(ctx, tmp_path):
+    """One pass of n = 2^14 wins the tuner's batch; few polynomials still run
+    in two passes on a tuned context, and on one that loads its choices."""
+    ctx.autotune(14, 14)
+    ctx.autotune_save(tmp_path / "tuned")
+    loaded = V.Context()
+    loaded.autotune_load(tmp_path / "tuned")
+    for c in (ctx, loaded):
+        assert c.tile_bits(14) != 14
+        for bits in (50, 60):
+            assert _transforms(c, 14, bits, 16, 0) == (2, 1)
+    loaded.close()

@@ -300,6 +300,13 @@ int vkhel_ext_autotune(struct vkhel_ctx *ctx, uint32_t logn_lo,
 			ctx->tile_bits2[logn] = saved_tb2;
 			return rc;
 		}
+		// n = 2^14 in one pass wins this batch; whether it wins another depends
+		// on its number and class, which the built-in choice goes by
+		// (tile_bits_for_tasks), on two passes of the built-in tile otherwise.
+		// (Kept as the tile of every call, 16 polynomials each way took 44 us at
+		// 60 bits against 16.5, a single call 27 against 17.6.)
+		if (logn == 14 && cands[best].tb == 14)
+			cands[best].tb = 0;
 		cands[best].apply(ctx, logn);
 	}
 	return VKHEL_OK;
