@@ -1523,8 +1523,14 @@ __attribute__((amdgpu_waves_per_eu(pm_waves(LOGN, TB)))) void k_ntt_pm(
 #pragma unroll
 			for (int e = 0; e < 8; e++) {
 				if constexpr (MC == kClassFp) {
-					// both spectra are doubles below 8q here; one operand of a
-					// product has to be below q/2
+					// Both spectra are doubles below B here.  One operand of a product
+					// has to be about q/2 at most (fp_mul_bound's unit of slack covers
+					// the 1/1024 more that fp_reduce leaves), and the product within
+					// what the inverse's rounds are planned for: not at 8q, 2057/1024
+					// q, but for every shape compiled here (at most 1991).
+					constexpr int B = fp_forward_bound<G, G::ROUNDS>();
+					static_assert(B <= kFpLimit && fp_mul_bound(B) <= kFpInverseRound,
+							"the product passes the inverse's entry bound");
 					const FpK fk{k.c.fq, k.c.fqinv};
 					v[e] = __builtin_bit_cast(uint64_t, fp_mulmod(
 							__builtin_bit_cast(double, v[e]), fp_reduce(
