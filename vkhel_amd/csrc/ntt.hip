@@ -155,7 +155,14 @@ static const std::array<FusedEntry, kFusedEntries> &fused_table() {
 			t[i].k[kClassGeneral] = fused_class_table<TB, kClassGeneral>()[i];
 			t[i].k[kClassMid] = fused_class_table<TB, kClassMid>()[i];
 			t[i].k[kClassSmall] = fused_class_table<TB, kClassSmall>()[i];
-			t[i].k[kClassFp] = fused_class_table<TB, kClassFp>()[i];
+			ClassKernels &fp = t[i].k[kClassFp], &small = t[i].k[kClassSmall];
+			fp = fused_class_table<TB, kClassFp>()[i];
+			if (!fp.fwd) {
+				fp.fwd = small.fwd;
+				fp.inv = small.inv;
+			}
+			fp.fwd_h = small.fwd_h;
+			fp.inv_h = small.inv_h;
 		}
 		return t;
 	}();

@@ -1562,9 +1562,6 @@ constexpr void set_passes(PassKernel k[2]) {
 	k[1] = k_ntt_pass<LG, PS, INV, TB, MC, (alt_k1(LG, TB) > 0 ? 1 : 0)>;
 }
 
-// The whole-polynomial two-pass kernels and the one-launch ones are tuning
-// modes that measured slower than the split passes at every size: moduli of
-// the double-precision class run the small class's there.
 // One-pass transforms that run with 32 words per thread (ntt_wide.h).
 constexpr bool wide_ok(int logn, int tb, int mc) {
 	return mc == kClassFp && logn == 14 && tb == 14;
@@ -1578,11 +1575,16 @@ constexpr bool both_ok(int logn, int tb) {
 
 template <int LG, int TB, int MC>
 constexpr ClassKernels class_kernels() {
-	constexpr int MC2 = MC == kClassFp ? (int) kClassSmall : MC;
-	constexpr int MC1 = LG <= TB ? MC : MC2;
+	// The whole-polynomial two-pass kernels and the one-launch ones are tuning
+	// modes that measured slower than the split passes at every size: moduli
+	// of the double-precision class run the small class's there (ntt.hip
+	// fused_table puts them in).
+	constexpr bool own = MC != kClassFp;
 	ClassKernels k{};
-	k.fwd = k_ntt_fused<LG, false, TB, MC1>;
-	k.inv = k_ntt_fused<LG, true, TB, MC1>;
+	if constexpr (own || LG <= TB) {
+		k.fwd = k_ntt_fused<LG, false, TB, MC>;
+		k.inv = k_ntt_fused<LG, true, TB, MC>;
+	}
 	if constexpr (wide_ok(LG, TB, MC)) {
 		k.wide_fwd = k_ntt_wide<LG, false>;
 		k.wide_inv = k_ntt_wide<LG, true>;
@@ -1598,8 +1600,10 @@ constexpr ClassKernels class_kernels() {
 	set_passes<LG, TB, MC, 2, true>(k.inv_b);
 	set_passes<LG, TB, MC, 1, true>(k.inv_a);
 	k.pm = k_ntt_pm<LG, TB, MC>;
-	k.fwd_h = k_ntt_handoff<LG, false, TB, MC2>;
-	k.inv_h = k_ntt_handoff<LG, true, TB, MC2>;
+	if constexpr (own) {
+		k.fwd_h = k_ntt_handoff<LG, false, TB, MC>;
+		k.inv_h = k_ntt_handoff<LG, true, TB, MC>;
+	}
 	return k;
 }
 
