@@ -133,12 +133,13 @@ int vkhel_ext_set_ntt_algo(struct vkhel_ctx *, int algo);
  * vkhel_ext_autotune times each compiled tile size, with both pass modes
  * (below), for every log2 n in [logn_lo, logn_hi] (3..20) on `batch`
  * synthetic polynomials (0: enough to fill the device) and keeps the
- * fastest per size on this context. */
+ * fastest per size on this context; where that is n = 2^14 in one pass, the
+ * built-in choice, which takes one pass by number and modulus. */
 int vkhel_ext_autotune(struct vkhel_ctx *, uint32_t logn_lo, uint32_t logn_hi,
 		uint32_t batch);
-/* Tile size (log2 words) in use for log2 n, or -1 on error.  (Untuned,
- * batches of n = 2^14 that fill the device run in one pass on 2^14 tiles
- * instead of the 2^12 tiles reported.) */
+/* Tile size (log2 words) in use for log2 n, or -1 on error.  (With the
+ * built-in choice, batches of n = 2^14 that fill the device run in one pass on
+ * 2^14 tiles instead of the 2^12 tiles reported.) */
 int vkhel_ext_tile_bits(struct vkhel_ctx *, uint32_t logn);
 /* tile_bits 11..14, or 0 for the built-in default. */
 int vkhel_ext_set_tile_bits(struct vkhel_ctx *, uint32_t logn, int tile_bits);

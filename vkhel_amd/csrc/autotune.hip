@@ -1,7 +1,7 @@
 // Autotuner for the fused NTT kernels.  For each transform size it times
-// every compiled tile size (2^11, 2^12, 2^13 words, i.e. the stage-fusion
-// split and workgroup shape of the two-pass path) in both pass modes on a
-// synthetic batch held in device memory, in interleaved rounds, and keeps
+// every compiled tile size (2^11 to 2^14 words, i.e. the stage-fusion split
+// and workgroup shape of the two-pass path) in its pass modes on a synthetic
+// batch held in device memory, in interleaved rounds, and keeps
 // the fastest forward+inverse pair for the context.  The reference has no counterpart: its kernels have one fixed
 // shape (64-thread workgroups, one dispatch per butterfly group).
 #include <algorithm>
@@ -240,9 +240,7 @@ int vkhel_ext_autotune(struct vkhel_ctx *ctx, uint32_t logn_lo,
 	// A 50-bit NTT prime (1 mod 2^21) and synthetic twiddles: timing does
 	// not depend on the values, only on the residues staying below q.
 	const uint64_t q = 1125899906826241ull;
-	hipStream_t s = ctx->stream;
 	for (uint32_t logn = logn_lo; logn <= logn_hi; logn++) {
-		const uint64_t n = 1ull << logn;
 		// only sizes above the smallest tile have more than one variant
 		if (logn <= 11)
 			continue;

@@ -181,8 +181,8 @@ struct TableGenArgs {
 };
 void table_gen_args(uint64_t n, uint64_t q, uint64_t w, TableGenArgs &g);
 // Writes both interleaved {w, Shoup companion} tables of n = 2^g.logn
-// entries (the layout tw_pos describes) on stream `st`.
-// and, unless `fp` is null, the 2n doubles of the double-precision class.
+// entries (the layout tw_pos describes) on stream `st` and, unless `fp` is
+// null, the 2n doubles of the double-precision class.
 hipError_t launch_gen_tables(const TableGenArgs &g, ulonglong2 *fwd,
 		ulonglong2 *inv, double *fp, hipStream_t st);
 uint64_t inv_mod_2_64(uint64_t q);
@@ -249,7 +249,7 @@ struct NttTask {
 	const ulonglong2 *tw2;
 };
 // 136 bytes of constants and five pointers; with 40 more the first launch of a
-// batch of 16384 tasks took 1.56 ms for 1.40 (MI355X, of which 0.31 on the
+// batch of 16384 tasks took 1.54 ms for 1.40 (MI355X; 0.29 of it on the
 // device).
 static_assert(sizeof(NttTask) <= 176, "tasks grew");
 

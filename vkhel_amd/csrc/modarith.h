@@ -55,14 +55,14 @@ __device__ __forceinline__ void ieee_mode_off(uint64_t &q, uint64_t &two_q) {
 			: "+s"(q), "+s"(two_q));
 }
 
-// csub for x < 2^63 and m <= 2^62 with nm = 2^64 - m given, in two
+// csub for x < 2m and m <= 2^62 with nm = 2^64 - m given, in two
 // instructions: d = x - m, and the smaller of x and |d| as double-precision
 // bit patterns (|.| clears bit 63, an input modifier).  Patterns without the
 // sign bit order as the integers they are.  For x >= m, |d| = d <= x; for
 // x < m the cleared d is 2^63 - (m - x) > x.  Patterns from 2^63 - 2^52 up
 // are NaNs, and v_min_f64 returns the operand that is none: there x is one
-// only if x >= m (result d), the cleared d only if x < m (result x), never
-// both.  Subnormals pass unchanged (double-precision subnormals are on), and
+// only if x >= m (result d, which is below m and no NaN), the cleared d only
+// if x < m (result x), never both.  Subnormals pass unchanged (double-precision subnormals are on), and
 // signaling NaNs too in a kernel that has called ieee_mode_off(); with IEEE mode
 // on they would come back quieted.
 // Measured on MI355X in issue slots of a 64-bit add: 1.9, against 3.8 for

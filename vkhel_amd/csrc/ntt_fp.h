@@ -10,7 +10,8 @@
 // need no offset in the difference, and a twiddle is one 8-byte double
 // instead of a 16-byte pair.  Measured on MI355X, split passes, 512 x 2^16
 // forward and inverse 434 -> 395 us (the passes are then bound by memory:
-// 5.4 TB/s), 512 x 2^14 119 -> 110, a single 2^16 call 23.0 -> 21.0.
+// 5.4 TB/s; 362 with their input streamed, batch.hip stream_input), 512 x 2^14
+// 119 -> 110, a single 2^16 call 23.0 -> 21.0.
 #pragma once
 
 #include "internal.h"

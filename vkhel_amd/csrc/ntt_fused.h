@@ -1,5 +1,5 @@
-// Stage-fused NTT engine for gfx950 (device templates).  Included by the
-// per-tile-size instantiation units ntt_fused_kt*.hip.
+// Stage-fused NTT engine for gfx950 (device templates).  Instantiated by
+// ntt_fused_inst.hip, once per tile size and modulus class.
 #pragma once
 
 #include <array>

@@ -10,7 +10,11 @@
 // low halves of all words first and the high halves after them through 66 KiB
 // of LDS, so two workgroups share a CU and one's loads and stores run beside
 // the other's arithmetic.
-// @@FIGURES@@
+// Measured on MI355X, forward + inverse, us, against eight words per thread:
+// 512 polynomials 89.5 -> 80.5, 2048 329 -> 295.  Not all of the arithmetic fits
+// the 128 registers: the compiler spills 34 values of the forward (92 bytes of
+// scratch per lane) and 6 of the inverse (28 bytes), and the forward's
+// spilled words show as 20% more written than the result holds.
 #pragma once
 
 namespace vk {
