@@ -45,6 +45,7 @@ Also reported, each with its own timing:
 """
 import argparse
 import ctypes
+import glob
 import json
 import os
 import sys
@@ -235,7 +236,7 @@ def batched_ntt(V, ctx, logn, primes, per_prime, steps, warmup, ev):
            "secs": secs, "gpu_ms": gpu_ms, "steps": steps, "fwd_ms": fwd_ms,
            "inv_ms": inv_ms,
            "gcoeff": 2 * npoly * n * steps / secs / 1e9,
-           "batches": (both, fwd, inv)}
+           "fwd_launches": fwd.shape()[0], "batches": (both, fwd, inv)}
     return res
 
 
@@ -864,21 +865,27 @@ def plain_polymul_n4096(V, ctx, runs=7):
             "bit_exact": ok}
 
 
-def traffic_from_profile(logn, npoly, tile_bits):
-    """HBM bytes per forward transform of the batch (both pass dispatches),
-    from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary of this
-    workload (scaled by the copy-kernel calibration recorded beside it), or
-    None when no summary of the same tile size exists."""
-    path = os.path.join(REPO, "profiles",
-                        f"ntt_fwd_n{1 << logn}_x{npoly}_tile{tile_bits}.json")
-    try:
+def traffic_from_profile(logn, npoly, kernels):
+    """HBM bytes per forward transform of the batch (all its dispatches), from
+    the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summaries of this workload
+    (scaled by the copy-kernel calibration recorded beside them), their time-
+    weighted VALU busy share, and the summaries' names.  One summary per tile
+    size; a transform may mix two (its passes' tiles are tuned apart).  None
+    three times unless every kernel is in one."""
+    found = {}
+    for path in sorted(glob.glob(os.path.join(
+            REPO, "profiles", f"ntt_fwd_n{1 << logn}_x{npoly}_tile*.json"))):
         with open(path) as f:
             prof = json.load(f)
-    except (OSError, ValueError):
-        return None, None
-    if prof.get("tile_bits") != tile_bits:
-        return None, prof
-    return prof.get("hbm_bytes_per_launch"), prof
+        for name, d in prof["per_dispatch"].items():
+            found.setdefault(name, (d, "profiles/" + os.path.basename(path)[:-4] + "md"))
+    if not all(k in found for k in kernels):
+        return None, None, None
+    ds = [found[k][0] for k in kernels]
+    us = sum(d["avg_us"] for d in ds)
+    return (round(sum(d["fetch_b"] + d["write_b"] for d in ds)),
+            round(sum(d["valu_busy"] * d["avg_us"] for d in ds) / us, 2),
+            " + ".join(sorted({found[k][1] for k in kernels})))
 
 
 def modulus_class(q):
@@ -906,10 +913,20 @@ def _alt_k1(logn, tb):
     return k + 1 if _split_ok(logn, tb, k + 1) else k - 1 if _split_ok(logn, tb, k - 1) else -1
 
 
-def fwd_kernel_names(logn, tile_bits, pass_mode, mc, split=0, tile_bits2=0):
+def forward_tile(logn, tile_bits, launches):
+    """The tile of a batch's forward transforms: the built-in choice for
+    n = 2^14 runs in one launch, on 2^14 words, where that pays."""
+    return 14 if logn == 14 and launches == 1 else tile_bits
+
+
+def fwd_kernel_names(logn, tile_bits, pass_mode, mc, split=0, tile_bits2=0, npoly=1):
     """The dispatches of one forward transform at this size and tuning for
     moduli of class mc (the last template argument of a pass kernel is 1 for
     the alternative stage split where the size has one)."""
+    if logn == tile_bits == 14 and mc == 3 and npoly > 256:  # more than CUs
+        return ["k_ntt_wide<14, false>"]
+    if mc == 3 and logn > tile_bits and pass_mode in (1, 3):
+        mc = 2  # the class has none of its own in these modes
     if logn <= tile_bits or pass_mode == 1:
         return [f"k_ntt_fused<{logn}, false, {tile_bits}, {mc}>"]
     if pass_mode == 3:
@@ -1005,7 +1022,8 @@ def main():
     r = batched_ntt(V, ctx, args.logn, args.primes, args.per_prime, args.steps,
                     args.warmup, ev)
     n, npoly = r["n"], r["npoly"]
-    alg_bytes = 16 * npoly * n + 16 * n * args.primes
+    # (a twiddle is one double below 2^50, a pair of words above)
+    alg_bytes = 16 * npoly * n + (8 if modulus_class(max(r["qs"])) == 3 else 16) * n * args.primes
     achieved = alg_bytes / (r["fwd_ms"] * 1e-3) / 1e9
     plain = plain_per_call(V, ctx, r, args.plain_polys)
     plain["speedup"] = round(r["gcoeff"] / plain["value"], 1)
@@ -1036,8 +1054,11 @@ def main():
         extra["map_unmap"] = map_unmap_leg(V, ctx)
 
     cpu = None if args.no_cpu else cpu_baseline(args.logn, qs, ws, V, ctx)
-    tb = ctx.tile_bits(args.logn)
-    traffic, prof = traffic_from_profile(args.logn, npoly, tb)
+    tb = forward_tile(args.logn, ctx.tile_bits(args.logn), r["fwd_launches"])
+    kernels = fwd_kernel_names(args.logn, tb, ctx.pass_mode(args.logn),
+                               modulus_class(max(qs)), ctx.split(args.logn),
+                               ctx.tile_bits2(args.logn), npoly)
+    traffic, valu_busy, profile = traffic_from_profile(args.logn, npoly, kernels)
     out = {
         "metric": "batched NTT Gcoeff/s & %HBM peak at N=2^16; served p50/p99 vs plain per-call",
         "value": round(r["gcoeff"], 3),
@@ -1059,17 +1080,12 @@ def main():
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
-                     "kernel": "forward NTT of the batch: " + " + ".join(
-                         fwd_kernel_names(args.logn, tb, ctx.pass_mode(args.logn),
-                                          modulus_class(max(qs)),
-                                          ctx.split(args.logn),
-                                          ctx.tile_bits2(args.logn))),
+                     "kernel": "forward NTT of the batch: " + " + ".join(kernels),
                      "kernel_ms": round(r["fwd_ms"], 4),
                      "inverse_kernel_ms": round(r["inv_ms"], 4),
                      "alg_bytes_per_launch": alg_bytes,
-                     "profile": (f"profiles/ntt_fwd_n{n}_x{npoly}_tile{tb}.md"
-                                 if prof else None),
-                     "profiled_valu_busy": prof.get("valu_busy") if prof and traffic else None},
+                     "profile": profile,
+                     "profiled_valu_busy": valu_busy},
         "plain_per_call": plain,
         "tile_bits": tuned,
         "pass_mode": modes,
