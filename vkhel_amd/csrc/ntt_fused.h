@@ -443,7 +443,9 @@ __device__ __forceinline__ double gload_tw(const double *p, uint32_t i) {
 	return *(gcdouble *) ((gcchar *) p + (i << 3));
 }
 
-// One padding word per 8 keeps the radix-8 access patterns conflict free.
+// One padding word per 8 spreads the radix-8 strides over the banks (not free of
+// conflicts: 128 conflict cycles per wave counted at n = 2^12, 32 LDS
+// instructions).
 __host__ __device__ __forceinline__ uint32_t pad(uint32_t l) {
 	return l + (l >> 3);
 }
