@@ -230,8 +230,9 @@ static bool default_passes(const vkhel_ctx *ctx, uint32_t logn) {
 	return pass_mode_of(ctx, logn) == 0 || pass_mode_of(ctx, logn) == 2;
 }
 
-// The tile for `ntasks` transforms at once.  Untuned n = 2^14 runs in one
-// pass on 2^14-word tiles where that fills the device: its time goes in steps
+// The tile for `ntasks` transforms at once.  n = 2^14 with the built-in choice
+// (untuned, or left to it by the tuner) runs in one pass on 2^14-word tiles
+// where that fills the device: its time goes in steps
 // of one CU-full of polynomials (one workgroup per CU, or two with 32 words
 // per thread, launch_fused_impl), the two passes' with their number.  Forward
 // + inverse on MI355X (256 CUs), us, moduli below 2^50, two passes / one of
